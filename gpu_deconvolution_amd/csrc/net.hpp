@@ -47,7 +47,9 @@ void launch_conv_out(const uint16_t* h, const uint16_t* x, Dims d, const float* 
 int launch_loss(const float* y, const float* t, long count, float* dy, double* partial, hipStream_t s);
 void launch_out_dgrad(const float* dy, Dims d, const float* small, float* dh, hipStream_t s);
 void launch_mask(const float* dh, const uint16_t* r, long count, uint16_t* g, hipStream_t s);
-// partial weight gradients, one row of (weights + biases) per (n, z) plane
+// weight gradients (net_wgrad.hip): wgrad_blocks(d) partial rows of (weights +
+// biases), then their sum
+int wgrad_blocks(Dims d);
 void launch_wgrad_in(const uint16_t* g, const uint16_t* x, Dims d, float* partial, hipStream_t s);
 void launch_wgrad_out(const float* dy, const uint16_t* h5, Dims d, float* partial, hipStream_t s);
 void launch_wgrad32(const uint16_t* g, const uint16_t* a, Dims d, float* partial, hipStream_t s);

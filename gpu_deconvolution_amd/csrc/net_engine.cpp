@@ -86,7 +86,7 @@ struct Engine {
             dy.alloc(sizeof(float) * nv);
             dh.alloc(sizeof(float) * kC * nv);
             g.alloc(sizeof(uint16_t) * kC * nv);
-            partial.alloc(sizeof(float) * (size_t)d.N * d.D * (kConv32 + kC));
+            partial.alloc(sizeof(float) * (size_t)wgrad_blocks(d) * (kConv32 + kC));
             lossPart.alloc(sizeof(double) * 1024);
         } else {
             r[0].alloc(sizeof(uint16_t) * kC * nv);  // relu scratch of the forward kernels
@@ -117,23 +117,23 @@ struct Engine {
         const long nv = d.voxels();
         const int nb = launch_loss(y.as<float>(), t, nv, dy.as<float>(), lossPart.as<double>(), s);
         float* G = grads.as<float>();
-        const int planes = d.N * d.D;
+        const int rows = wgrad_blocks(d);
         // layer 6
         launch_wgrad_out(dy.as<float>(), h[4].as<uint16_t>(), d, partial.as<float>(), s);
-        launch_reduce_partials(partial.as<float>(), planes, w_size(5) + b_size(5), G + off_w(5), s);
+        launch_reduce_partials(partial.as<float>(), rows, w_size(5) + b_size(5), G + off_w(5), s);
         launch_out_dgrad(dy.as<float>(), d, small.as<float>(), dh.as<float>(), s);
         // layers 5 .. 2
         for (int l = 4; l >= 1; --l) {
             launch_mask(dh.as<float>(), r[l].as<uint16_t>(), nv * kC, g.as<uint16_t>(), s);
             launch_wgrad32(g.as<uint16_t>(), h[l - 1].as<uint16_t>(), d, partial.as<float>(), s);
-            launch_reduce_partials(partial.as<float>(), planes, kConv32 + kC, G + off_w(l), s);
+            launch_reduce_partials(partial.as<float>(), rows, kConv32 + kC, G + off_w(l), s);
             launch_conv32_dgrad(g.as<uint16_t>(), d, wt.as<uint16_t>() + (size_t)(l - 1) * kConv32, dh.as<float>(),
                                 s);
         }
         // layer 1 (mask: h1 = relu(a1))
         launch_mask(dh.as<float>(), h[0].as<uint16_t>(), nv * kC, g.as<uint16_t>(), s);
         launch_wgrad_in(g.as<uint16_t>(), x.as<uint16_t>(), d, partial.as<float>(), s);
-        launch_reduce_partials(partial.as<float>(), planes, w_size(0) + b_size(0), G + off_w(0), s);
+        launch_reduce_partials(partial.as<float>(), rows, w_size(0) + b_size(0), G + off_w(0), s);
         std::vector<double> part(nb);
         FMVD_HIP(hipMemcpyAsync(part.data(), lossPart.p, sizeof(double) * nb, hipMemcpyDeviceToHost, s));
         FMVD_HIP(hipStreamSynchronize(s));

@@ -12,9 +12,7 @@
 // K = 27 taps x 32 input channels with v_mfma_f32_32x32x16_bf16 (A = 32
 // consecutive voxels x 16 channels loaded straight from the activation
 // layout, B = 16 channels x 32 outputs from the block's LDS copy of the
-// layer weights).  The weight gradient of those layers is the same GEMM with
-// voxels as the reduction dimension, staged through LDS in channel-major
-// order.  The 2->32 input layer and the 32->1 output layer have too few
+// layer weights).  The weight gradients are in net_wgrad.hip.  The 2->32 input layer and the 32->1 output layer have too few
 // channels for MFMA tiles and run on the VALU, still with FP32 accumulation.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -24,28 +22,10 @@
 
 #include "hip_check.hpp"
 #include "net.hpp"
+#include "net_device.hpp"
 
 namespace fmvd {
 namespace net {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-__device__ __forceinline__ float bf2f(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
-// round to nearest even (finite inputs)
-__device__ __forceinline__ uint16_t f2bf(float f)
-{
-    const uint32_t u = __float_as_uint(f);
-    return (uint16_t)((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
-}
-
-struct Geo {
-    int N, D, H, W;  // batch, depth, height, width
-    __device__ __forceinline__ long vox(int n, int z, int y, int x) const
-    {
-        return (((long)n * D + z) * H + y) * W + x;
-    }
-};
 
 // ------------------------------------------------------------ MFMA check
 // D = A (32 x 16) * B (16 x 32) for a unit test of the operand layout:
@@ -273,159 +253,6 @@ __global__ void mask_kernel(const float* __restrict__ dh, const uint16_t* __rest
     gout[i] = (r[i] & 0x7FFFu) != 0 && !(r[i] & 0x8000u) ? f2bf(dh[i]) : (uint16_t)0;
 }
 
-// Weight gradient of the two small layers on the VALU: one block per (n, z)
-// plane.  Per output row y the block stages the row's gradients (W x COUT,
-// FP32) in LDS, then, one at a time, each of the 9 input rows
-// (z + dz - 1, y + dy - 1) over x = -1 .. W (FP32); thread t accumulates the
-// products e = t, t + 256, ... of dW[k][co][ci] = sum_v g[v][co] a[v + off(k)][ci]
-// whose tap uses the staged row, plus the bias sums.  Layer 1: a = x
-// (CIN 2), g bf16 (COUT 32).  Layer 6: a = h5 (CIN 32), g = dy FP32 (COUT 1).
-// Requires W <= kMaxW.
-constexpr int kMaxW = 256;
-template <int CIN, int COUT, bool GF32>
-__global__ __launch_bounds__(256) void wgrad_small_kernel(const void* __restrict__ gv, const uint16_t* __restrict__ a,
-                                                          Geo g, float* __restrict__ partial)
-{
-    constexpr int NW = 27 * COUT * CIN, NP = NW + COUT, PER = (NP + 255) / 256;
-    __shared__ float gs[kMaxW * COUT];          // [x][co]
-    __shared__ float as[(kMaxW + 2) * CIN];     // [x + 1][ci]
-    const int n = blockIdx.x / g.D, z = blockIdx.x % g.D;
-    float acc[PER];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) acc[j] = 0.f;
-    for (int y = 0; y < g.H; ++y) {
-        __syncthreads();
-        for (int e = threadIdx.x; e < g.W * COUT; e += 256) {
-            const long v = g.vox(n, z, y, e / COUT);
-            gs[e] = GF32 ? static_cast<const float*>(gv)[v * COUT + e % COUT]
-                         : bf2f(static_cast<const uint16_t*>(gv)[v * COUT + e % COUT]);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {  // bias sums need only the gradients
-            const int e = threadIdx.x + 256 * j;
-            if (e >= NW && e < NP) {
-                float s = 0.f;
-                for (int x = 0; x < g.W; ++x) s += gs[x * COUT + (e - NW)];
-                acc[j] += s;
-            }
-        }
-        for (int row = 0; row < 9; ++row) {
-            const int zz = z + row / 3 - 1, yy = y + row % 3 - 1;
-            const bool rowok = zz >= 0 && zz < g.D && yy >= 0 && yy < g.H;  // block-uniform
-            if (!rowok) continue;
-            __syncthreads();
-            for (int e = threadIdx.x; e < (g.W + 2) * CIN; e += 256) {
-                const int xx = e / CIN - 1, ci = e % CIN;
-                as[e] = (xx >= 0 && xx < g.W) ? bf2f(a[g.vox(n, zz, yy, xx) * CIN + ci]) : 0.f;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < PER; ++j) {
-                const int e = threadIdx.x + 256 * j;
-                if (e < NW) {
-                    const int k = e / (COUT * CIN), co = (e / CIN) % COUT, ci = e % CIN;
-                    if (k / 3 != row) continue;
-                    const float* ar = as + (k % 3) * CIN + ci;  // voxel x + dx - 1 -> ar[x * CIN]
-                    float s = 0.f;
-                    for (int x = 0; x < g.W; ++x) s += gs[x * COUT + co] * ar[x * CIN];
-                    acc[j] += s;
-                }
-            }
-        }
-    }
-    float* p = partial + (long)blockIdx.x * NP;
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const int e = threadIdx.x + 256 * j;
-        if (e < NP) p[e] = acc[j];
-    }
-}
-
-// MFMA weight gradient of a 32 -> 32 layer: one block per (n, z) plane, 4
-// waves; wave w accumulates taps k = w, w+4, ... (<= 7 taps x 16 floats).
-// Per 16-voxel chunk of an output row the block stages g (16 vox x 32 co)
-// and the 9 shifted input rows (18 vox x 32 ci, x0-1 .. x0+16) in LDS in
-// channel-major order, so each lane's A (8 voxels of one co) and B (8 voxels
-// of one ci) operands are contiguous.  Bias sums come from the same tiles.
-__global__ __launch_bounds__(256) void wgrad_mfma_kernel(const uint16_t* __restrict__ gin,
-                                                         const uint16_t* __restrict__ a, Geo g,
-                                                         float* __restrict__ partial)
-{
-    __shared__ __attribute__((aligned(16))) uint16_t gt[32][16];  // [co][voxel]
-    __shared__ uint16_t at[9][32][24];       // [row][ci][x - x0 + 1], 18 used (+ pad)
-    __shared__ float bias[4][32];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int n = blockIdx.x / g.D, z = blockIdx.x % g.D;
-    const int m = lane & 31, kh = lane >> 5;
-    f32x16 acc[7];
-#pragma unroll
-    for (int j = 0; j < 7; ++j) acc[j] = f32x16{};
-    float bsum = 0.f;
-    for (int y = 0; y < g.H; ++y)
-        for (int x0 = 0; x0 < g.W; x0 += 16) {
-            __syncthreads();
-            // stage g: 16 voxels x 32 co, transposed
-            for (int e = threadIdx.x; e < 16 * 32; e += 256) {
-                const int vx = e / 32, co = e % 32;
-                const int xx = x0 + vx;
-                gt[co][vx] = xx < g.W ? gin[g.vox(n, z, y, xx) * 32 + co] : (uint16_t)0;
-            }
-            // stage the 9 shifted input rows: 18 voxels x 32 ci each, transposed
-            for (int e = threadIdx.x; e < 9 * 18 * 32; e += 256) {
-                const int row = e / (18 * 32), vx = (e / 32) % 18, ci = e % 32;
-                const int zz = z + row / 3 - 1, yy = y + row % 3 - 1, xx = x0 + vx - 1;
-                const bool ok = zz >= 0 && zz < g.D && yy >= 0 && yy < g.H && xx >= 0 && xx < g.W;
-                at[row][ci][vx] = ok ? a[g.vox(n, zz, yy, xx) * 32 + ci] : (uint16_t)0;
-            }
-            __syncthreads();
-            // A = g^T: lane (m = co, kh) holds voxels 8 kh .. 8 kh + 7
-            const bf16x8 av = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&gt[m][8 * kh]));
-            if (wave == 0 && kh == 0) {
-#pragma unroll
-                for (int j = 0; j < 16; ++j) bsum += bf2f(gt[m][j]);
-            }
-#pragma unroll
-            for (int j = 0; j < 7; ++j) {
-                const int k = wave + 4 * j;
-                if (k < 27) {
-                    // B = shifted input: lane (n = ci, kh) holds voxels x0 + 8 kh + j' + dx - 1
-                    const int row = k / 3, dx = k % 3;
-                    bf16x8 bv;
-#pragma unroll
-                    for (int jj = 0; jj < 8; ++jj) bv[jj] = __builtin_bit_cast(__bf16, at[row][m][8 * kh + jj + dx]);
-                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc[j], 0, 0, 0);
-                }
-            }
-        }
-    // D[co][ci]: lane holds ci = m, co = 8(r/4) + 4 kh + r%4
-    float* p = partial + (long)blockIdx.x * (27 * 32 * 32 + 32);
-#pragma unroll
-    for (int j = 0; j < 7; ++j) {
-        const int k = wave + 4 * j;
-        if (k < 27) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int co = 8 * (r / 4) + 4 * kh + (r % 4);
-                p[(k * 32 + co) * 32 + m] = acc[j][r];
-            }
-        }
-    }
-    if (wave == 0 && kh == 0) bias[0][m] = bsum;
-    __syncthreads();
-    if (threadIdx.x < 32) p[27 * 32 * 32 + threadIdx.x] = bias[0][threadIdx.x];
-}
-
-// sum partials[nb][count] -> out[count] (FP64 accumulation)
-__global__ void reduce_partials_kernel(const float* __restrict__ partial, int nb, int count, float* __restrict__ out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    double s = 0.0;
-    for (int b = 0; b < nb; ++b) s += (double)partial[(long)b * count + i];
-    out[i] = (float)s;
-}
-
 // Adam on FP32 master parameters; also refreshes the bf16 copies used by
 // the kernels.  Bias-corrected (Kingma & Ba 2015).
 __global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ gr, float* __restrict__ m,
@@ -502,7 +329,6 @@ __global__ void scale_out_kernel(const float* __restrict__ yr, Geo r, int H, int
 }
 
 // ------------------------------------------------------------ launchers
-static inline Geo geo(Dims d) { return Geo{d.N, d.D, d.H, d.W}; }
 static inline unsigned nblk(long n, int t) { return (unsigned)((n + t - 1) / t); }
 
 void launch_mfma_layout_test(const uint16_t* A, const uint16_t* B, float* D, hipStream_t s)
@@ -571,28 +397,6 @@ void launch_out_dgrad(const float* dy, Dims d, const float* small, float* dh, hi
 void launch_mask(const float* dh, const uint16_t* r, long count, uint16_t* g, hipStream_t s)
 {
     mask_kernel<<<nblk(count, 256), 256, 0, s>>>(dh, r, count, g);
-    FMVD_LAUNCH_CHECK();
-}
-void launch_wgrad_in(const uint16_t* g, const uint16_t* x, Dims d, float* partial, hipStream_t s)
-{
-    if (d.W > kMaxW) throw_msg("network: volume width above 256");
-    wgrad_small_kernel<2, 32, false><<<d.N * d.D, 256, 0, s>>>(g, x, geo(d), partial);
-    FMVD_LAUNCH_CHECK();
-}
-void launch_wgrad_out(const float* dy, const uint16_t* h5, Dims d, float* partial, hipStream_t s)
-{
-    if (d.W > kMaxW) throw_msg("network: volume width above 256");
-    wgrad_small_kernel<32, 1, true><<<d.N * d.D, 256, 0, s>>>(dy, h5, geo(d), partial);
-    FMVD_LAUNCH_CHECK();
-}
-void launch_wgrad32(const uint16_t* g, const uint16_t* a, Dims d, float* partial, hipStream_t s)
-{
-    wgrad_mfma_kernel<<<d.N * d.D, 256, 0, s>>>(g, a, geo(d), partial);
-    FMVD_LAUNCH_CHECK();
-}
-void launch_reduce_partials(const float* partial, int nb, int count, float* out, hipStream_t s)
-{
-    reduce_partials_kernel<<<nblk(count, 256), 256, 0, s>>>(partial, nb, count, out);
     FMVD_LAUNCH_CHECK();
 }
 void launch_adam(float* p, const float* g, float* m, float* v, int count, float lr, int step, hipStream_t s)

@@ -136,3 +136,22 @@ def test_tiled_inference_equals_whole_volume(fm):
     a, b = whole.download(), tiled.download()
     assert np.isfinite(a).all() and a.min() >= 1e-3
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 1, 8, 32), (1, 3, 9, 33), (1, 4, 17, 31), (1, 5, 16, 66),
+                                   (3, 90, 4, 5)])
+def test_gradients_at_tile_edges(fm, shape):
+    """Volumes of one voxel, of whole tiles, of a tile and a remainder on each
+    axis, and of more (sample, plane) pairs than CUs.  Tolerance: five times
+    the bfloat16 spacing 2^-8, since a stored activation may round to the
+    neighbouring bfloat16 value."""
+    params, x, t = make_problem(13, shape)
+    _, y, loss, g = run_gpu(fm, params, x, t)
+    loss_o, grads_o, y_o = oracle_batch(params, x, t)
+    assert relL2(y, y_o) < 2e-2
+    assert abs(loss - loss_o) < 2e-2 * loss_o
+    gg = unflat(g)
+    for l in range(onet.LAYERS):
+        for i in range(2):
+            d, n = np.linalg.norm(gg[l][i] - grads_o[l][i]), np.linalg.norm(grads_o[l][i])
+            assert d <= 2e-2 * n + 1e-7, (l, i, d, n)
