@@ -37,16 +37,22 @@ void launch_prep_input(const uint16_t* const* d_views, int nviews, Dims d, const
 void launch_prep_region(const uint16_t* const* d_views, int nviews, int D, int H, int W, int z0, int y0, int x0,
                         Dims r, float inv_scale, uint16_t* x, hipStream_t s);
 void launch_pack_weights(const float* params, uint16_t* wf, uint16_t* wt, float* small, hipStream_t s);
-void launch_conv_in(const uint16_t* x, Dims d, const float* small, const float* params, uint16_t* h, hipStream_t s);
-void launch_conv32_fwd(const uint16_t* in, Dims d, const uint16_t* wf_layer, const float* bias, uint16_t* rout,
+void launch_conv_in(const uint16_t* x, Dims d, const float* small, const float* params, uint16_t* h,
+                    uint32_t* relu, hipStream_t s);
+// 32 -> 32 layers (net_conv32.hip).  relu: one dword per voxel with the bits
+// "channel's relu output > 0", written by the forward (null: not wanted) and
+// read by the gradients of the layers above; dgrad adds to dh (stored only while
+// keep_dh) and writes the masked bf16 gradient of the layer below to gout.
+void launch_conv32_fwd(const uint16_t* in, Dims d, const uint16_t* wf_layer, const float* bias, uint32_t* relu,
                        uint16_t* hout, hipStream_t s);
-void launch_conv32_dgrad(const uint16_t* g, Dims d, const uint16_t* wt_layer, float* dh, hipStream_t s);
+void launch_conv32_dgrad(const uint16_t* g, Dims d, const uint16_t* wt_layer, const uint32_t* relu, float* dh,
+                         bool keep_dh, uint16_t* gout, hipStream_t s);
 void launch_conv_out(const uint16_t* h, const uint16_t* x, Dims d, const float* small, const float* params, float* y,
                      hipStream_t s);
 // loss partial sums (FP64, one per block of the returned count) and dy
 int launch_loss(const float* y, const float* t, long count, float* dy, double* partial, hipStream_t s);
-void launch_out_dgrad(const float* dy, Dims d, const float* small, float* dh, hipStream_t s);
-void launch_mask(const float* dh, const uint16_t* r, long count, uint16_t* g, hipStream_t s);
+void launch_out_dgrad(const float* dy, Dims d, const float* small, const uint32_t* relu, float* dh, uint16_t* gout,
+                      hipStream_t s);
 // weight gradients (net_wgrad.hip): wgrad_blocks(d) partial rows of (weights +
 // biases), then their sum
 int wgrad_blocks(Dims d);

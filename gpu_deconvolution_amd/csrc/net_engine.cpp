@@ -25,8 +25,8 @@ struct Engine {
     DeviceBuffer partial, lossPart;
     // activations for the current shape
     Dims cur{0, 0, 0, 0};
-    DeviceBuffer x, y, dy, dh, g;
-    DeviceBuffer h[5], r[5];
+    DeviceBuffer x, y, dy, dh, g[2];
+    DeviceBuffer h[5], relu[5];
     int step = 0;
     bool packed = false;
 
@@ -82,14 +82,12 @@ struct Engine {
         const int nh = training ? 5 : 2;
         for (int i = 0; i < nh; ++i) h[i].alloc(sizeof(uint16_t) * kC * nv);
         if (training) {
-            for (int i = 0; i < 5; ++i) r[i].alloc(sizeof(uint16_t) * kC * nv);
+            for (int i = 0; i < 5; ++i) relu[i].alloc(sizeof(uint32_t) * nv);
             dy.alloc(sizeof(float) * nv);
             dh.alloc(sizeof(float) * kC * nv);
-            g.alloc(sizeof(uint16_t) * kC * nv);
+            for (auto& b : g) b.alloc(sizeof(uint16_t) * kC * nv);
             partial.alloc(sizeof(float) * (size_t)wgrad_blocks(d) * (kConv32 + kC));
             lossPart.alloc(sizeof(double) * 1024);
-        } else {
-            r[0].alloc(sizeof(uint16_t) * kC * nv);  // relu scratch of the forward kernels
         }
         cur = d;
     }
@@ -100,12 +98,12 @@ struct Engine {
         pack(s);
         const float* P = params.as<float>();
         const uint16_t* X = x.as<uint16_t>();
-        launch_conv_in(X, d, small.as<float>(), P, h[0].as<uint16_t>(), s);
+        launch_conv_in(X, d, small.as<float>(), P, h[0].as<uint16_t>(), training ? relu[0].as<uint32_t>() : nullptr, s);
         for (int l = 1; l <= 4; ++l) {
             const uint16_t* in = training ? h[l - 1].as<uint16_t>() : h[(l - 1) & 1].as<uint16_t>();
             uint16_t* out = training ? h[l].as<uint16_t>() : h[l & 1].as<uint16_t>();
-            uint16_t* rr = training ? r[l].as<uint16_t>() : r[0].as<uint16_t>();
-            launch_conv32_fwd(in, d, wf.as<uint16_t>() + (size_t)(l - 1) * kConv32, P + off_b(l), rr, out, s);
+            launch_conv32_fwd(in, d, wf.as<uint16_t>() + (size_t)(l - 1) * kConv32, P + off_b(l),
+                              training ? relu[l].as<uint32_t>() : nullptr, out, s);
         }
         const uint16_t* h5 = training ? h[4].as<uint16_t>() : h[0].as<uint16_t>();
         launch_conv_out(h5, X, d, small.as<float>(), P, y.as<float>(), s);
@@ -121,18 +119,19 @@ struct Engine {
         // layer 6
         launch_wgrad_out(dy.as<float>(), h[4].as<uint16_t>(), d, partial.as<float>(), s);
         launch_reduce_partials(partial.as<float>(), rows, w_size(5) + b_size(5), G + off_w(5), s);
-        launch_out_dgrad(dy.as<float>(), d, small.as<float>(), dh.as<float>(), s);
-        // layers 5 .. 2
+        uint16_t* gc = g[0].as<uint16_t>();
+        uint16_t* gn = g[1].as<uint16_t>();
+        launch_out_dgrad(dy.as<float>(), d, small.as<float>(), relu[4].as<uint32_t>(), dh.as<float>(), gc, s);
+        // layers 5 .. 2; each input gradient writes the next layer's masked gradient
         for (int l = 4; l >= 1; --l) {
-            launch_mask(dh.as<float>(), r[l].as<uint16_t>(), nv * kC, g.as<uint16_t>(), s);
-            launch_wgrad32(g.as<uint16_t>(), h[l - 1].as<uint16_t>(), d, partial.as<float>(), s);
+            launch_wgrad32(gc, h[l - 1].as<uint16_t>(), d, partial.as<float>(), s);
             launch_reduce_partials(partial.as<float>(), rows, kConv32 + kC, G + off_w(l), s);
-            launch_conv32_dgrad(g.as<uint16_t>(), d, wt.as<uint16_t>() + (size_t)(l - 1) * kConv32, dh.as<float>(),
-                                s);
+            launch_conv32_dgrad(gc, d, wt.as<uint16_t>() + (size_t)(l - 1) * kConv32, relu[l - 1].as<uint32_t>(),
+                                dh.as<float>(), l > 1, gn, s);
+            std::swap(gc, gn);
         }
-        // layer 1 (mask: h1 = relu(a1))
-        launch_mask(dh.as<float>(), h[0].as<uint16_t>(), nv * kC, g.as<uint16_t>(), s);
-        launch_wgrad_in(g.as<uint16_t>(), x.as<uint16_t>(), d, partial.as<float>(), s);
+        // layer 1
+        launch_wgrad_in(gc, x.as<uint16_t>(), d, partial.as<float>(), s);
         launch_reduce_partials(partial.as<float>(), rows, w_size(0) + b_size(0), G + off_w(0), s);
         std::vector<double> part(nb);
         FMVD_HIP(hipMemcpyAsync(part.data(), lossPart.p, sizeof(double) * nb, hipMemcpyDeviceToHost, s));

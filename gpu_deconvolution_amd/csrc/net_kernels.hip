@@ -7,13 +7,10 @@
 // 32->32 layer are [tap][cout][cin] bf16 (tap = (dz*3 + dy)*3 + dx reads
 // voxel (z+dz-1, y+dy-1, x+dx-1); zero padding at the volume faces).
 //
-// The four 32->32 layers (98% of the work) run on MFMA: one wavefront
-// computes a 32-voxel x 32-channel output tile as an implicit GEMM over
-// K = 27 taps x 32 input channels with v_mfma_f32_32x32x16_bf16 (A = 32
-// consecutive voxels x 16 channels loaded straight from the activation
-// layout, B = 16 channels x 32 outputs from the block's LDS copy of the
-// layer weights).  The weight gradients are in net_wgrad.hip.  The 2->32 input layer and the 32->1 output layer have too few
-// channels for MFMA tiles and run on the VALU, still with FP32 accumulation.
+// The four 32->32 layers (98% of the work) run on MFMA (net_conv32.hip), their
+// weight gradients and those of the edge layers too (net_wgrad.hip).  The
+// 2->32 input layer and the 32->1 output layer have too few channels for MFMA
+// tiles and run on the VALU, still with FP32 accumulation.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -75,10 +72,17 @@ __global__ void prep_input_kernel(const uint16_t* const* __restrict__ views, int
     x[2 * (n * per + i) + 1] = f2bf(o * k);
 }
 
-// Layer 1 (2 -> 32), VALU: h1 = relu(conv(x, W1) + b1); W1 is FP32 [27][32][2]
-// (bf16-rounded values).  One thread per voxel.
+// The edge layers run on the VALU.
+
+// Layer 1 (2 -> 32): h1 = relu(conv(x, W1) + b1); W1 is FP32 [27][32][2]
+// (bf16-rounded values).  One thread per voxel; relu (if wanted): the bits h1 > 0.
+// Bound by the VALU: 27 x 32 x 3 instructions a voxel (two products, rounded
+// separately, and their sum) are 553 us at 8 x 64 x 128 x 128, measured 634; reading the
+// weights through scalar loads, or walking planes with 96 sums a thread to
+// read a neighbour once, measured 656 and 734.
 __global__ void conv_in_kernel(const uint16_t* __restrict__ x, Geo g, const float* __restrict__ w,
-                               const float* __restrict__ b, uint16_t* __restrict__ h)
+                               const float* __restrict__ b, uint16_t* __restrict__ h,
+                               uint32_t* __restrict__ relu)
 {
     __shared__ float ws[27 * 32 * 2 + 32];
     for (int i = threadIdx.x; i < 27 * 64 + 32; i += blockDim.x) ws[i] = i < 27 * 64 ? w[i] : b[i - 27 * 64];
@@ -100,99 +104,98 @@ __global__ void conv_in_kernel(const uint16_t* __restrict__ x, Geo g, const floa
         for (int c = 0; c < 32; ++c) acc[c] += x0 * ws[(k * 32 + c) * 2] + x1 * ws[(k * 32 + c) * 2 + 1];
     }
     uint16_t* o = h + (n * per + i) * 32;
+    uint32_t pos = 0;
 #pragma unroll
-    for (int c = 0; c < 32; ++c) o[c] = f2bf(fmaxf(acc[c], 0.f));
+    for (int c = 0; c < 32; ++c) {
+        const uint16_t r = f2bf(fmaxf(acc[c], 0.f));
+        if (r) pos |= 1u << c;
+        o[c] = r;
+    }
+    if (relu) relu[n * per + i] = pos;
 }
 
-// Layer 6 (32 -> 1), VALU: y = conv(h5, W6) + b6 + (x0 + x1) / 2 (FP32 out).
-__global__ void conv_out_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ x, Geo g,
-                                const float* __restrict__ w, const float* __restrict__ b, float* __restrict__ y)
+// Layer 6 (32 -> 1): y = conv(h5, W6) + b6 + (x0 + x1) / 2 (FP32 out).  A block
+// walks the planes p of a kOY x kOX column, one voxel per thread: the plane with its
+// halo is staged in LDS (the next one loads meanwhile), and each of a thread's 9
+// neighbours in it is read and converted once for its three taps dz, whose sums belong to
+// the outputs p + 1, p, p - 1; the weights are uniform and come through scalar
+// loads.  An output sums in the order dz, dy, dx, channel.  One voxel per thread with
+// 27 x 64 bytes from L1 and the weights from LDS took 843 us at 8 x 64 x 128 x 128; this 425,
+// of which the VALU's 1152 instructions a voxel are 246.
+constexpr int kOY = 8, kOX = 32, kOHX = kOX + 2, kOHV = (kOY + 2) * kOHX, kOPitch = 40;
+constexpr int kOPieces = (kOHV * 4 + 255) / 256, kOPlane = (kOY + 2) * kOPitch * 64;
+__global__ __launch_bounds__(256) void conv_out_kernel(const uint16_t* __restrict__ h, const uint32_t* __restrict__ x,
+                                                       Geo g, const float* __restrict__ w,
+                                                       const float* __restrict__ b, float* __restrict__ y, int nseg)
 {
-    __shared__ float ws[27 * 32];
-    for (int i = threadIdx.x; i < 27 * 32; i += blockDim.x) ws[i] = w[i];
-    __syncthreads();
-    const long per = (long)g.D * g.H * g.W;
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int n = blockIdx.y;
-    if (i >= per) return;
-    const int xx = (int)(i % g.W), yy = (int)((i / g.W) % g.H), zz = (int)(i / ((long)g.W * g.H));
-    float acc = b[0];
-    for (int k = 0; k < 27; ++k) {
-        const int z = zz + k / 9 - 1, yv = yy + (k / 3) % 3 - 1, xi = xx + k % 3 - 1;
-        if (z < 0 || z >= g.D || yv < 0 || yv >= g.H || xi < 0 || xi >= g.W) continue;
-        const uint4* hv = reinterpret_cast<const uint4*>(h + g.vox(n, z, yv, xi) * 32);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint4 u = hv[q];
-            const uint32_t wds[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int c = q * 8 + 2 * j;
-                acc += bf2f((uint16_t)(wds[j] & 0xFFFFu)) * ws[k * 32 + c];
-                acc += bf2f((uint16_t)(wds[j] >> 16)) * ws[k * 32 + c + 1];
-            }
-        }
-    }
-    const long v = n * per + i;
-    y[v] = acc + 0.5f * (bf2f(x[2 * v]) + bf2f(x[2 * v + 1]));
-}
+    __shared__ __attribute__((aligned(16))) char planes[2][kOPlane];
+    const int nx = (g.W + kOX - 1) / kOX, ny = (g.H + kOY - 1) / kOY;
+    const unsigned bid = xcd_block(blockIdx.x, gridDim.x);
+    const int seg = bid % nseg, tile = bid / nseg, n = tile / (nx * ny);
+    const int y0 = (tile / nx) % ny * kOY, x0 = tile % nx * kOX;
+    const int za = (int)((long)g.D * seg / nseg), zb = (int)((long)g.D * (seg + 1) / nseg);
+    const int row = threadIdx.x / kOX, col = threadIdx.x % kOX;
 
-// --------------------------------------------------------- MFMA conv 32->32
-// Block: 4 wavefronts; wave w computes row (n, z, y0 + w) of 32-voxel tiles
-// x0 = 32 t.  Weights [27][32 cout][32 cin] bf16 are staged in LDS.
-// MODE 0 (forward):  r = relu(acc + b);  hout = hin + r  (bf16 stores of r, hout)
-// MODE 1 (dgrad):    dh[v] += acc  (FP32, in place; weights given transposed)
-template <int MODE>
-__global__ __launch_bounds__(256) void conv32_mfma_kernel(const uint16_t* __restrict__ in, Geo g,
-                                                          const uint16_t* __restrict__ wt, const float* __restrict__ b,
-                                                          const uint16_t* __restrict__ hin, uint16_t* __restrict__ rout,
-                                                          uint16_t* __restrict__ hout, float* __restrict__ dh)
-{
-    __shared__ uint4 wl[27 * 32 * 32 * 2 / 16];  // 27 taps x 32 x 32 bf16
-    {
-        const uint4* src = reinterpret_cast<const uint4*>(wt);
-        for (int i = threadIdx.x; i < 27 * 32 * 32 * 2 / 16; i += 256) wl[i] = src[i];
-    }
+    uint4 pre[kOPieces];
+    auto load = [&](int z) {
+#pragma unroll
+        for (int i = 0; i < kOPieces; ++i) {
+            const int e = threadIdx.x + 256 * i, v = e >> 2, yy = y0 + v / kOHX - 1, xx = x0 + v % kOHX - 1;
+            pre[i] = make_uint4(0, 0, 0, 0);
+            if (v < kOHV && yy >= 0 && yy < g.H && xx >= 0 && xx < g.W)
+                pre[i] = reinterpret_cast<const uint4*>(h + g.vox(n, z, yy, xx) * 32)[e & 3];
+        }
+    };
+    auto store = [&](int z) {
+#pragma unroll
+        for (int i = 0; i < kOPieces; ++i) {
+            const int e = threadIdx.x + 256 * i, v = e >> 2, yy = v / kOHX, xx = v % kOHX;
+            if (v < kOHV)
+                *reinterpret_cast<uint4*>(planes[z & 1] + (yy * kOPitch + xx) * 64 + (((e & 3) ^ slot_swizzle(xx)) << 4)) =
+                    pre[i];
+        }
+    };
+    const float bias = b[0];
+    float a0 = bias, a1 = bias, a2 = bias;
+    const int pa = max(za - 1, 0);
+    load(pa);
+    store(pa);
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int rows = (g.H + 3) / 4;
-    const int n = blockIdx.x / (g.D * rows);
-    const int rem = blockIdx.x % (g.D * rows);
-    const int z = rem / rows, y = (rem % rows) * 4 + wave;
-    if (y >= g.H) return;  // wave-uniform; no block barrier follows
-    const int m = lane & 31, kh = lane >> 5;  // tile voxel / K half of this lane
-    const uint16_t* wl16 = reinterpret_cast<const uint16_t*>(wl);
-    for (int x0 = 0; x0 < g.W; x0 += 32) {
-        f32x16 acc = {};
-        for (int k = 0; k < 27; ++k) {
-            const int zz = z + k / 9 - 1, yy = y + (k / 3) % 3 - 1, xx = x0 + m + k % 3 - 1;
-            const bool ok = zz >= 0 && zz < g.D && yy >= 0 && yy < g.H && xx >= 0 && xx < g.W;
-            const uint16_t* ip = in + g.vox(n, ok ? zz : 0, ok ? yy : 0, ok ? xx : 0) * 32;
+    for (int p = pa; p <= zb; ++p) {
+        const bool next = p < zb && p + 1 < g.D;
+        if (next) load(p + 1);
+        if (p < g.D) {
+#pragma unroll 1
+            for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
-            for (int kc = 0; kc < 2; ++kc) {
-                const int c0 = 16 * kc + 8 * kh;
-                uint4 av = ok ? *reinterpret_cast<const uint4*>(ip + c0) : make_uint4(0, 0, 0, 0);
-                const uint4 bv = *reinterpret_cast<const uint4*>(wl16 + (k * 32 + m) * 32 + c0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av),
-                                                              __builtin_bit_cast(bf16x8, bv), acc, 0, 0, 0);
-            }
-        }
-        // lane holds D[voxel mv][channel m] for mv = 8(r/4) + 4 kh + r%4
+                for (int dx = 0; dx < 3; ++dx) {
+                    const char* v = planes[p & 1] + ((row + dy) * kOPitch + col + dx) * 64;
+                    const float* wk = w + (dy * 3 + dx) * 32;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int mv = 8 * (r / 4) + 4 * kh + (r % 4);
-            const int xx = x0 + mv;
-            if (xx >= g.W) continue;
-            const long o = g.vox(n, z, y, xx) * 32 + m;
-            if constexpr (MODE == 0) {
-                const float rv = fmaxf(acc[r] + b[m], 0.f);
-                const uint16_t rb = f2bf(rv);
-                rout[o] = rb;
-                hout[o] = f2bf(bf2f(hin[o]) + bf2f(rb));
-            } else {
-                dh[o] += acc[r];
-            }
+                    for (int q = 0; q < 4; ++q) {
+                        const uint4 u = *reinterpret_cast<const uint4*>(v + ((q ^ slot_swizzle(col + dx)) << 4));
+                        const uint32_t wds[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) {
+                            const float f = bf2f((uint16_t)(wds[j / 2] >> (16 * (j & 1))));
+                            a0 += f * wk[8 * q + j];
+                            a1 += f * wk[9 * 32 + 8 * q + j];
+                            a2 += f * wk[18 * 32 + 8 * q + j];
+                        }
+                    }
+                }
         }
+        if (next) store(p + 1);
+        const int z = p - 1, yy = y0 + row, xx = x0 + col;
+        if (z >= za && yy < g.H && xx < g.W) {
+            const long v = g.vox(n, z, yy, xx);
+            const uint32_t u = x[v];
+            y[v] = a2 + 0.5f * (bf2f((uint16_t)u) + bf2f((uint16_t)(u >> 16)));
+        }
+        a2 = a1;
+        a1 = a0;
+        a0 = bias;
+        if (next) __syncthreads();
     }
 }
 
@@ -217,9 +220,11 @@ __global__ void loss_kernel(const float* __restrict__ y, const float* __restrict
     if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// dh5[v][c] = sum_k dy[v - off(k)] W6[k][c]  (FP32 out)
+// dh5[v][c] = sum_k dy[v - off(k)] W6[k][c]  (FP32 out), and the masked bf16
+// gradient of layer 5 (relu: its bits r > 0)
 __global__ void out_dgrad_kernel(const float* __restrict__ dy, Geo g, const float* __restrict__ w,
-                                 float* __restrict__ dh)
+                                 const uint32_t* __restrict__ relu, float* __restrict__ dh,
+                                 uint16_t* __restrict__ gout)
 {
     __shared__ float ws[27 * 32];
     for (int i = threadIdx.x; i < 27 * 32; i += blockDim.x) ws[i] = w[i];
@@ -240,17 +245,13 @@ __global__ void out_dgrad_kernel(const float* __restrict__ dy, Geo g, const floa
         for (int c = 0; c < 32; ++c) acc[c] += d * ws[k * 32 + c];
     }
     float* o = dh + (n * per + i) * 32;
+    uint16_t* go = gout + (n * per + i) * 32;
+    const uint32_t bits = relu[n * per + i];
 #pragma unroll
-    for (int c = 0; c < 32; ++c) o[c] = acc[c];
-}
-
-// g = bf16(dh * (r > 0))
-__global__ void mask_kernel(const float* __restrict__ dh, const uint16_t* __restrict__ r, long count,
-                            uint16_t* __restrict__ gout)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= count) return;
-    gout[i] = (r[i] & 0x7FFFu) != 0 && !(r[i] & 0x8000u) ? f2bf(dh[i]) : (uint16_t)0;
+    for (int c = 0; c < 32; ++c) {
+        o[c] = acc[c];
+        go[c] = (bits >> c) & 1 ? f2bf(acc[c]) : (uint16_t)0;
+    }
 }
 
 // Adam on FP32 master parameters; also refreshes the bf16 copies used by
@@ -355,30 +356,22 @@ void launch_pack_weights(const float* params, uint16_t* wf, uint16_t* wt, float*
     pack_weights_kernel<<<nblk(4 * kConv32, 256), 256, 0, s>>>(params, wf, wt, small);
     FMVD_LAUNCH_CHECK();
 }
-void launch_conv_in(const uint16_t* x, Dims d, const float* small, const float* params, uint16_t* h, hipStream_t s)
+void launch_conv_in(const uint16_t* x, Dims d, const float* small, const float* params, uint16_t* h,
+                    uint32_t* relu, hipStream_t s)
 {
     const long per = (long)d.D * d.H * d.W;
-    conv_in_kernel<<<dim3(nblk(per, 256), d.N), 256, 0, s>>>(x, geo(d), small, params + off_b(0), h);
-    FMVD_LAUNCH_CHECK();
-}
-static inline unsigned conv32_blocks(Dims d) { return (unsigned)((long)d.N * d.D * ((d.H + 3) / 4)); }
-void launch_conv32_fwd(const uint16_t* in, Dims d, const uint16_t* wf_layer, const float* bias, uint16_t* rout,
-                       uint16_t* hout, hipStream_t s)
-{
-    conv32_mfma_kernel<0><<<conv32_blocks(d), 256, 0, s>>>(in, geo(d), wf_layer, bias, in, rout, hout, nullptr);
-    FMVD_LAUNCH_CHECK();
-}
-void launch_conv32_dgrad(const uint16_t* g, Dims d, const uint16_t* wt_layer, float* dh, hipStream_t s)
-{
-    conv32_mfma_kernel<1><<<conv32_blocks(d), 256, 0, s>>>(g, geo(d), wt_layer, nullptr, nullptr, nullptr, nullptr,
-                                                           dh);
+    conv_in_kernel<<<dim3(nblk(per, 256), d.N), 256, 0, s>>>(x, geo(d), small, params + off_b(0), h, relu);
     FMVD_LAUNCH_CHECK();
 }
 void launch_conv_out(const uint16_t* h, const uint16_t* x, Dims d, const float* small, const float* params, float* y,
                      hipStream_t s)
 {
-    const long per = (long)d.D * d.H * d.W;
-    conv_out_kernel<<<dim3(nblk(per, 256), d.N), 256, 0, s>>>(h, x, geo(d), small + 27 * 64, params + off_b(5), y);
+    // segments of about 16 planes: a segment reads two planes beyond its ends
+    const int nseg = (d.D + 15) / 16;
+    const long blocks = (long)d.N * ((d.H + kOY - 1) / kOY) * ((d.W + kOX - 1) / kOX) * nseg;
+    if (blocks > 0x7fffffffL) throw_msg("network: volume too large");
+    conv_out_kernel<<<(unsigned)blocks, 256, 0, s>>>(h, reinterpret_cast<const uint32_t*>(x), geo(d), small + 27 * 64,
+                                                     params + off_b(5), y, nseg);
     FMVD_LAUNCH_CHECK();
 }
 int launch_loss(const float* y, const float* t, long count, float* dy, double* partial, hipStream_t s)
@@ -388,15 +381,11 @@ int launch_loss(const float* y, const float* t, long count, float* dy, double* p
     FMVD_LAUNCH_CHECK();
     return nb;
 }
-void launch_out_dgrad(const float* dy, Dims d, const float* small, float* dh, hipStream_t s)
+void launch_out_dgrad(const float* dy, Dims d, const float* small, const uint32_t* relu, float* dh, uint16_t* gout,
+                      hipStream_t s)
 {
     const long per = (long)d.D * d.H * d.W;
-    out_dgrad_kernel<<<dim3(nblk(per, 256), d.N), 256, 0, s>>>(dy, geo(d), small + 27 * 64, dh);
-    FMVD_LAUNCH_CHECK();
-}
-void launch_mask(const float* dh, const uint16_t* r, long count, uint16_t* g, hipStream_t s)
-{
-    mask_kernel<<<nblk(count, 256), 256, 0, s>>>(dh, r, count, g);
+    out_dgrad_kernel<<<dim3(nblk(per, 256), d.N), 256, 0, s>>>(dy, geo(d), small + 27 * 64, relu, dh, gout);
     FMVD_LAUNCH_CHECK();
 }
 void launch_adam(float* p, const float* g, float* m, float* v, int count, float lr, int step, hipStream_t s)

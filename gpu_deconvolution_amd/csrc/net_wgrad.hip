@@ -116,14 +116,16 @@ __device__ __forceinline__ bf16x8 read_tr(const char* lds, int off0, int off1)
 // delivers 1.14 operands (1 KiB each, 8 cycles) per 32-cycle MFMA and SIMD: the matrix
 // cores and the LDS are about equally busy.
 constexpr int kNT = 7;  // taps per wavefront
-constexpr int kWgradLds = 4 * kNT * 16 * 64 * 4;  // the second row group's sums at the end
-static_assert(3 * kHaloBytes + kTileBytes <= kWgradLds);
+// A ring of four planes and two tiles: the next step's go where no wavefront of this
+// step reads, so a step needs one barrier.
+constexpr int kWgradLds = 4 * kHaloBytes + 2 * kTileBytes;
+static_assert(4 * kNT * 16 * 64 * 4 <= kWgradLds);  // the second row group's sums at the end
 __global__ __launch_bounds__(kWThreads, 2) void wgrad32_kernel(const uint16_t* __restrict__ gin,
                                                                const uint16_t* __restrict__ a, Geo g, int steps,
                                                                float* __restrict__ partial)
 {
     __shared__ __attribute__((aligned(16))) char lds[kWgradLds];
-    char* const tile = lds + 3 * kHaloBytes;
+    char* const tiles = lds + 4 * kHaloBytes;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int w4 = wave & 3, rows = (wave >> 2) * (kWY / 2);
     const unsigned b = xcd_block(blockIdx.x, gridDim.x);
@@ -153,10 +155,10 @@ __global__ __launch_bounds__(kWThreads, 2) void wgrad32_kernel(const uint16_t* _
             __syncthreads();
             for (int dz = 0; dz < 3; ++dz) {
                 load_halo(rh, a, g, c, z + dz - 1);
-                store_halo(lds + (z + dz + 2) % 3 * kHaloBytes, rh);
+                store_halo(lds + ((z + dz - 1) & 3) * kHaloBytes, rh);
             }
             load_tile(rt, gin, g, c, z);
-            store_tile(tile, rt);
+            store_tile(tiles + (z & 1) * kTileBytes, rt);
             __syncthreads();
         }
         const bool next = s + 1 < s1 && z + 1 < g.D;
@@ -168,8 +170,9 @@ __global__ __launch_bounds__(kWThreads, 2) void wgrad32_kernel(const uint16_t* _
 #pragma unroll
         for (int j = 0; j < kNT; ++j) {
             const int k = min(w4 + 4 * j, 26);
-            tap[j] = (z + k / 9 + 2) % 3 * kHaloBytes + k / 3 % 3 * (kPitch * kVB);
+            tap[j] = ((z + k / 9 - 1) & 3) * kHaloBytes + k / 3 % 3 * (kPitch * kVB);
         }
+        const char* tile = tiles + (z & 1) * kTileBytes;
 #pragma unroll
         for (int y = 0; y < kWY / 2; ++y)
 #pragma unroll
@@ -184,9 +187,8 @@ __global__ __launch_bounds__(kWThreads, 2) void wgrad32_kernel(const uint16_t* _
                 }
             }
         if (next) {
-            __syncthreads();
-            store_halo(lds + (z + 2) % 3 * kHaloBytes, rh);
-            store_tile(tile, rt);
+            store_halo(lds + ((z + 2) & 3) * kHaloBytes, rh);
+            store_tile(tiles + ((z + 1) & 1) * kTileBytes, rt);
             __syncthreads();
         }
     }
@@ -407,8 +409,9 @@ __global__ __launch_bounds__(kWThreads, 4) void wgrad_out_kernel(const uint32_t*
 }
 
 // Sum partials[nb][count] -> out[count] in FP64: a block takes 32 columns and
-// deals the rows to 8 groups of 32 lanes (one thread per column left 108
-// blocks with nb dependent loads each: 127 us at 512 x 27 680, against 26).
+// deals the rows to 8 groups of 32 lanes.  (One thread per column left 108
+// blocks with nb dependent loads each; over the six layers of a step with 512
+// rows the mean was 127 us a launch, against 9.)
 __global__ __launch_bounds__(256) void reduce_partials_kernel(const float* __restrict__ partial, int nb, int count,
                                                               float* __restrict__ out)
 {
