@@ -148,12 +148,35 @@ struct Engine {
         packed = false;
     }
 
+    // Tiles of fmvd_net_infer: the halo is the receptive field, and the longest
+    // extent is halved (thirds, ...) until a tile with its halo has at most 16 M
+    // voxels (136 bytes of activations each: 2.2 GB).  Voxels computed per voxel
+    // of a 1024 x 2048 x 2048 volume: 1.16, of a 96 x 300 x 260 one: 1 (tiles of
+    // 128 x 224 x 224 with a halo of 16: 1.63 and 1.24).
+    static constexpr int kReach = 6;
+    static void tiles(int D, int H, int W, int t[3])
+    {
+        const int n[3] = {D, H, W};
+        int parts[3] = {1, 1, 1};
+        for (;;) {
+            double voxels = 1.0;
+            int longest = 0;
+            for (int a = 0; a < 3; ++a) {
+                t[a] = (n[a] + parts[a] - 1) / parts[a];
+                voxels *= parts[a] > 1 ? std::min(n[a], t[a] + 2 * kReach) : n[a];
+                if (t[a] > t[longest]) longest = a;
+            }
+            if (voxels <= (double)(16 << 20) || t[longest] <= 32) return;
+            ++parts[longest];
+        }
+    }
+
     // Tile-wise inference: interior tiles of at most (tz, ty, tx) with a halo
     // of `halo` voxels on every side that lies inside the volume.  The
     // receptive field of the network is 6 voxels, so with halo >= 6 the
     // result equals whole-volume inference.
     void infer(const uint16_t* const* d_views, int nviews, int D, int H, int W, float scale, float floor_value,
-               float* out, hipStream_t s, int tz = 128, int ty = 224, int tx = 224, int halo = 16)
+               float* out, hipStream_t s, int tz, int ty, int tx, int halo)
     {
         const float inv = 1.0f / scale;
         for (int z0 = 0; z0 < D; z0 += tz)
@@ -276,7 +299,10 @@ int fmvd_net_prep_input(const unsigned short* const* d_views, int nviews, int N,
 int fmvd_net_infer(struct fmvd_net* n, const unsigned short* const* d_views, int nviews, int D, int H, int W,
                    float scale, float floor_value, float* d_out, void* stream)
 {
-    return fmvd_net_infer_tiled(n, d_views, nviews, D, H, W, scale, floor_value, 128, 224, 224, 16, d_out, stream);
+    int t[3] = {1, 1, 1};
+    if (D > 0 && H > 0 && W > 0) fmvd::net::Engine::tiles(D, H, W, t);
+    return fmvd_net_infer_tiled(n, d_views, nviews, D, H, W, scale, floor_value, t[0], t[1], t[2],
+                                fmvd::net::Engine::kReach, d_out, stream);
 }
 
 int fmvd_net_infer_tiled(struct fmvd_net* n, const unsigned short* const* d_views, int nviews, int D, int H, int W,

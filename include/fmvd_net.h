@@ -48,8 +48,8 @@ int fmvd_net_adam(struct fmvd_net *net, float lr, void *stream);
 int fmvd_net_prep_input(const unsigned short *const *d_views, int nviews, int N, int D, int H, int W,
                         const float *d_inv_scales, void *d_x, void *stream);
 /* Warm start of one volume: d_out (float D*H*W, device) = max(scale * net(views / scale), floor_value),
- * computed tile-wise (interior tiles of at most 128 x 224 x 224 voxels with a
- * 16-voxel halo inside the volume; identical to whole-volume inference).
+ * computed tile-wise (tiles of at most 16 M voxels with the network's 6-voxel
+ * reach as halo; identical to whole-volume inference).
  * d_views: nviews device pointers (device array). */
 int fmvd_net_infer(struct fmvd_net *net, const unsigned short *const *d_views, int nviews, int D, int H, int W,
                    float scale, float floor_value, float *d_out, void *stream);
