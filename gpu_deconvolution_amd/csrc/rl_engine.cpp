@@ -569,35 +569,69 @@ template <typename S> struct Plan {
         for (int k = 0; k <= iterations; ++k) errs[k] = h[2 * k + 1] > 0 ? std::sqrt(h[2 * k] / h[2 * k + 1]) : 0.0;
     }
 
+    // Planes per batch of the streaming pipeline: one chunk (the launches of a
+    // larger batch are no larger), so that a short stream already overlaps its
+    // host copies with the device, unless the caller set the batch.
+    int stream_planes() const
+    {
+        return batchCap > 0 ? batchCap : std::min(batch_planes(), std::max(chunk_planes(), nStreams));
+    }
+
+    // The pipeline's staging, two slots: kept from run to run (allocating and
+    // pinning it on every call took 8 times as long as deconvolving 40 planes of
+    // 512^2), at most two batches of samples and results, freed with the plan.
+    struct Staging {
+        DeviceBuffer in, out, est;
+        PinnedBuffer hin, hout, hest;
+        Event up, run, done;
+    };
+    std::unique_ptr<Staging> staging[2];
+    std::unique_ptr<Stream> down;
+
     // fmvd_deconvolve.impl.cpp:205-300, as a double-buffered batch pipeline:
     // while batch i computes on the compute stream, the host pulls batch i+1
-    // from the datasource and uploads it on the copy stream, and pushes batch
-    // i-1's results to the datasink.  Planes are pulled and pushed in z order.
+    // from the datasource and uploads it on the copy stream, and batch i-1's
+    // results are downloaded on a third stream and pushed to the datasink.  Planes
+    // are pulled and pushed in z order.
     void deconvolve_planes(int iterations)
     {
         if (!source || !sink) throw_msg("datasource and datasink must be set");
         if (iterations < 0) throw_msg("negative iteration count");
         FMVD_HIP(hipSetDevice(device));
         if (lookahead > 0) return deconvolve_planes_bounded(iterations);
-        const int nb = batch_planes();
+        try {
+            stream_batches(iterations);
+        } catch (...) {
+            // no copy may be in flight on the staging that the next run fills
+            (void)hipStreamSynchronize(copy->s);
+            (void)hipStreamSynchronize(compute->s);
+            if (down) (void)hipStreamSynchronize(down->s);
+            throw;
+        }
+    }
+
+    void stream_batches(int iterations)
+    {
+        const int nb = stream_planes();
         const size_t pl = plane();
         const size_t inBytes = sizeof(S) * pl * nViews * (size_t)nb;
-        DeviceBuffer din[2], dout, dest;
-        PinnedBuffer hin[2], hout[2], hest[2];
-        Event up[2], done[2];
-        for (int k = 0; k < 2; ++k) {
-            din[k].alloc(inBytes);
-            hin[k].alloc(inBytes);
-            hout[k].alloc(sizeof(S) * pl * nb);
-            if (esink) hest[k].alloc(sizeof(float) * pl * nb);
+        if (!down) down.reset(new Stream());
+        for (auto& st : staging) {
+            if (!st) st.reset(new Staging());
+            st->in.alloc(inBytes);
+            st->hin.alloc(inBytes);
+            st->out.alloc(sizeof(S) * pl * nb);
+            st->hout.alloc(sizeof(S) * pl * nb);
+            if (esink) {
+                st->est.alloc(sizeof(float) * pl * nb);
+                st->hest.alloc(sizeof(float) * pl * nb);
+            }
         }
-        dout.alloc(sizeof(S) * pl * nb);
-        if (esink) dest.alloc(sizeof(float) * pl * nb);
         ensure_work(nb);
 
         std::vector<S*> hviews[2];
         for (int k = 0; k < 2; ++k)
-            for (int v = 0; v < nViews; ++v) hviews[k].push_back(hin[k].as<S>() + (size_t)v * nb * pl);
+            for (int v = 0; v < nViews; ++v) hviews[k].push_back(staging[k]->hin.template as<S>() + (size_t)v * nb * pl);
         bool exhausted = false;
         auto fill = [&](int slot) -> int {
             int n = 0;
@@ -612,16 +646,16 @@ template <typename S> struct Plan {
         };
         auto send = [&](int slot, int n) {
             for (int v = 0; v < nViews; ++v)
-                FMVD_HIP(hipMemcpyAsync(din[slot].as<S>() + (size_t)v * nb * pl, hviews[slot][v],
+                FMVD_HIP(hipMemcpyAsync(staging[slot]->in.template as<S>() + (size_t)v * nb * pl, hviews[slot][v],
                                         sizeof(S) * pl * n, hipMemcpyHostToDevice, copy->s));
-            FMVD_HIP(hipEventRecord(up[slot].e, copy->s));
+            FMVD_HIP(hipEventRecord(staging[slot]->up.e, copy->s));
         };
         int zout = 0;
         auto drain = [&](int slot, int n) {
-            FMVD_HIP(hipEventSynchronize(done[slot].e));
+            FMVD_HIP(hipEventSynchronize(staging[slot]->done.e));
             for (int j = 0; j < n; ++j) {
-                if (esink) esink(hest[slot].as<float>() + (size_t)j * pl, zout, euser);
-                sink(hout[slot].as<S>() + (size_t)j * pl);
+                if (esink) esink(staging[slot]->hest.template as<float>() + (size_t)j * pl, zout, euser);
+                sink(staging[slot]->hout.template as<S>() + (size_t)j * pl);
                 ++zout;
             }
         };
@@ -635,16 +669,18 @@ template <typename S> struct Plan {
         std::vector<const S*> vv(nViews);
         for (;;) {
             hipStream_t cs = compute->s;
-            FMVD_HIP(hipStreamWaitEvent(cs, up[slot].e, 0));
-            for (int v = 0; v < nViews; ++v) vv[v] = din[slot].as<S>() + (size_t)v * nb * pl;
-            run_batch(vv.data(), (long)pl, cnt[slot], iterations, nullptr, 0, dout.as<S>(),
-                      esink ? dest.as<float>() : nullptr, (long)pl, cs);
-            FMVD_HIP(hipMemcpyAsync(hout[slot].p, dout.p, sizeof(S) * pl * cnt[slot],
-                                    hipMemcpyDeviceToHost, cs));
+            FMVD_HIP(hipStreamWaitEvent(cs, staging[slot]->up.e, 0));
+            for (int v = 0; v < nViews; ++v) vv[v] = staging[slot]->in.template as<S>() + (size_t)v * nb * pl;
+            Staging& st = *staging[slot];
+            run_batch(vv.data(), (long)pl, cnt[slot], iterations, nullptr, 0, st.out.template as<S>(),
+                      esink ? st.est.template as<float>() : nullptr, (long)pl, cs);
+            FMVD_HIP(hipEventRecord(st.run.e, cs));
+            FMVD_HIP(hipStreamWaitEvent(down->s, st.run.e, 0));
+            FMVD_HIP(hipMemcpyAsync(st.hout.p, st.out.p, sizeof(S) * pl * cnt[slot], hipMemcpyDeviceToHost, down->s));
             if (esink)
-                FMVD_HIP(hipMemcpyAsync(hest[slot].p, dest.p, sizeof(float) * pl * cnt[slot],
-                                        hipMemcpyDeviceToHost, cs));
-            FMVD_HIP(hipEventRecord(done[slot].e, cs));
+                FMVD_HIP(hipMemcpyAsync(st.hest.p, st.est.p, sizeof(float) * pl * cnt[slot], hipMemcpyDeviceToHost,
+                                        down->s));
+            FMVD_HIP(hipEventRecord(st.done.e, down->s));
             const int ns = slot ^ 1;
             if (prev) drain(ns, cnt[ns]);
             cnt[ns] = exhausted ? 0 : fill(ns);

@@ -53,8 +53,11 @@ struct fmvd_plan_cuda_8;
  * Normalises h_Kernel[v] in place (as the reference does), copies the
  * weights and retains the callbacks.  nstreams >= 1 is the minimum number of
  * planes kept in flight; the plan processes planes in batches of at least
- * that many (fmvd_set_batch_planes_cuda_*), sized from a 2 GiB device budget
- * by default. */
+ * that many (fmvd_set_batch_planes_cuda_*): by default one chunk
+ * (fmvd_set_chunk_planes_cuda_*) of a stream of host planes, and as many planes
+ * of a GPU-resident volume as a 2 GiB device budget holds.  The staging of a stream
+ * (two batches of samples and results, on the device and pinned) stays with the
+ * plan. */
 struct fmvd_plan_cuda_16 *fmvd_initialize_cuda_16(
     int dataH, int dataW, float const *const *h_Weights, float **h_Kernel, int kernelH,
     int kernelW, fmvd_psf_type iteration_type, int nViews, int nstreams,

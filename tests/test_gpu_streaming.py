@@ -46,3 +46,19 @@ def test_lookahead_call_order_and_results(fm, D, L):
     for kind, ok in calls:
         held += 1 if (kind == "get" and ok) else (-1 if kind == "put" else 0)
         assert 0 <= held <= L
+
+
+@pytest.mark.parametrize("D", [1, 4, 11])
+def test_staging_kept_between_runs(fm, D):
+    """One plan, runs of changing length, with and without the estimate sink,
+    against a single-batch plan: batches of 2 planes, so 11 planes reuse each slot."""
+    V, dh, dw, k = 2, 40, 52, 9
+    data, kernels, weights = make_case(D, V, dh, dw, k, k, 16, seed=70 + D)
+    planes = [[data[z, v] for v in range(V)] for z in range(D)]
+    with fm.Deconvolver(dh, dw, list(weights), [x.copy() for x in kernels], batch_planes=64) as dec:
+        out, est = dec.run(planes, 3, want_estimate=True)
+    with fm.Deconvolver(dh, dw, list(weights), [x.copy() for x in kernels], nstreams=1, chunk_planes=2) as dec:
+        for n, sink in ((D, False), (D, True), (0, True), (max(1, D - 3), True), (D, True)):
+            o, e = dec.run(planes[:n], 3, want_estimate=sink)
+            assert np.array_equal(o, out[:n])
+            assert not (sink and n) or np.array_equal(e, est[:n])
