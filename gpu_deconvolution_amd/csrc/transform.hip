@@ -66,6 +66,13 @@ __device__ __forceinline__ void fetch_pair(const S* __restrict__ src, int w, int
     }
 }
 
+// a b + c d, each operation rounded.
+__device__ __forceinline__ double mul_add(double a, double b, double c, double d)
+{
+#pragma clang fp contract(off)
+    return a * b + c * d;
+}
+
 // One output sample at plane z of target column (x, y); axy[a] holds
 // m[4a] x + m[4a+1] y (the first sum of the fixed operation order).  FP64
 // with no contraction:
@@ -119,15 +126,13 @@ __device__ __forceinline__ S transform_sample(const S* __restrict__ src, int w, 
     return (S)0;
 }
 
-// A thread computes kGZ consecutive target planes of one (x, y) column; a
-// workgroup holds 64 x 4 columns.  The trilinear fetches read the source
-// straight from global memory (two samples per load).  Under a rotation the
-// 64 lanes of a wavefront walk diagonally through the source, so a source
-// cache line is used by outputs that are neighbours in 3D, not along one
-// target row: workgroups are therefore taken in supertiles of kSX x kSY x kSZ
-// workgroups (128 x 32 x 32 target voxels, about 1.5 MB of source), numbered
-// x fastest, then y, then z, with each XCD given a contiguous range, so the
-// supertiles in flight on one XCD keep their source rows in its L2.
+// General kernel: any map.  A thread computes kGZ consecutive target planes of one
+// (x, y) column; a workgroup holds 64 x 4 columns.  The trilinear fetches read the source
+// straight from global memory (two samples per load).  Workgroups are taken in
+// supertiles of kSX x kSY x kSZ workgroups (128 x 32 x 32 target voxels, about 1.5 MB
+// of source), numbered x fastest, then y, then z, with each XCD given a
+// contiguous range, so the supertiles in flight on one XCD keep their source
+// rows in its L2.
 constexpr int kGX = 64, kGY = 4, kGZ = 8;
 constexpr unsigned kSX = 2, kSY = 8, kSZ = 4, kSuper = kSX * kSY * kSZ;
 
@@ -139,7 +144,7 @@ __device__ __forceinline__ unsigned xcd_block(unsigned bid, unsigned nblocks)
 }
 
 template <typename S>
-__global__ __launch_bounds__(256) void transform_kernel(const S* __restrict__ src, int w, int h, int d,
+__global__ __launch_bounds__(256) void transform_general_kernel(const S* __restrict__ src, int w, int h, int d,
                                                         S* __restrict__ dst, int tw, int th, int z0, int nz,
                                                         Mat12 M, unsigned nbx, unsigned nby, unsigned nsx,
                                                         unsigned nsy)
@@ -155,12 +160,200 @@ __global__ __launch_bounds__(256) void transform_kernel(const S* __restrict__ sr
     const int y = (int)by * kGY + (int)(threadIdx.x / kGX);
     if (x >= tw || y >= th) return;
     const double xd = (double)x, yd = (double)y;
-    const double axy[3] = {M.m[0] * xd + M.m[1] * yd, M.m[4] * xd + M.m[5] * yd, M.m[8] * xd + M.m[9] * yd};
+    const double axy[3] = {mul_add(M.m[0], xd, M.m[1], yd), mul_add(M.m[4], xd, M.m[5], yd),
+                           mul_add(M.m[8], xd, M.m[9], yd)};
     const int zb = z0 + (int)bz * kGZ, ze = min(zb + kGZ, z0 + nz);
     if (zb >= ze) return;
     S* out = dst + ((size_t)(zb - z0) * th + y) * tw + x;
     const size_t pstride = (size_t)th * tw;
     for (int z = zb; z < ze; ++z, out += pstride) *out = transform_sample<S>(src, w, h, d, M, axy, z);
+}
+
+// ------------------------------------------------------------------ box kernel
+// A workgroup computes a cube of kT^3 target voxels.  It stages the bounding box of the
+// cube's texels (3.8 texels an output at +-15 degrees about each axis) in LDS with
+// coalesced loads, zero outside the volume, and gathers from there without
+// bounds checks.  Gathering straight from global memory costs the texture path
+// about one cycle per lane and load, whatever the lanes' arrangement (48 L1 accesses a
+// load; 64 x 1, 32 x 2, 16 x 4 and 8 x 8 voxels ran alike, as did aligned loads):
+// 190 cycles for 64 outputs, against about 40 for the four LDS reads.  1024^2 x
+// 512 voxels of 16 bits under such maps: 3.06 ms gathered, 1.36 ms here (1.6 TB/s
+// of 2.1 GB); the VALU is about 90 % busy, 45 of the 65 instructions a sample FP64,
+// conversions or byte shifts (4.4 cycles each, the 32-bit ones 2.5).  301 x 257 x 129
+// voxels of 8 bits into 333 x 270 x 141: 95 -> 60 us.
+//
+// The arithmetic is FP64 with fewer operations than the definition: the
+// coordinates as one FMA on a sum per (x, y) column, lerps as v + f (v' - v).  The result
+// differs from the definition's by at most `guard` output units (transform_guard),
+// so a sample farther than that from a rounding boundary is the definition's, and
+// any other is evaluated by transform_sample.
+constexpr int kT = 16, kBoxThreads = 512;
+constexpr unsigned kBoxSuper = 4;  // supertiles of 4^3 cubes, about 1.7 MB of source
+
+struct BoxMap {
+    double guard;
+    int ny, nz;         // rows and planes of the box
+    int pieces;         // pieces staged per row
+    int pitch, plane;   // bytes from row to row and plane to plane
+    int step, step_y, step_z;  // rows staged at a time: floor(threads / pieces) = step_z ny + step_y
+    unsigned magic_pieces;     // ceil(2^16 / pieces): i / pieces = i magic >> 16 for i < 512, pieces <= 150
+    unsigned nx, nby, nsx, nsy;  // cubes, and supertiles, along x and y
+};
+
+__device__ __forceinline__ double lerp(double a, double b, double f) { return fma(f, b - a, a); }
+// Samples x, x + 1 of a staged row, `shift` bytes into the word at LDS address `at`, interpolated.
+template <typename S> __device__ __forceinline__ double lerp_row(uint32_t at, uint32_t shift, double f)
+{
+    typedef uint32_t two __attribute__((ext_vector_type(2), aligned(4)));
+    const two t = *reinterpret_cast<__attribute__((address_space(3))) const two*>(at);
+    const uint32_t u = __builtin_amdgcn_alignbyte(t.y, t.x, shift);
+    constexpr uint32_t bits = 8 * sizeof(S), mask = (1u << bits) - 1u;
+    return lerp((double)(u & mask), (double)(u >> bits & mask), f);
+}
+__device__ __forceinline__ uint32_t lds_address(const void* p)
+{
+    return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
+}
+
+// The bytes of a piece from sample (x, y, z) on, zero where outside the volume.
+template <typename S, typename P>
+__device__ __forceinline__ P load_piece(const S* __restrict__ src, int w, int h, int d, int x, int y, int z)
+{
+    constexpr int n = sizeof(P) / sizeof(S);
+    P p{};
+    if (y < 0 || y >= h || z < 0 || z >= d || x + n <= 0 || x >= w) return p;
+    const S* row = src + ((size_t)z * h + y) * w;
+    if (x >= 0 && x + n <= w) {
+        if constexpr (sizeof(P) == 16) p = *reinterpret_cast<const P*>(row + x);
+        else __builtin_memcpy(&p, row + x, sizeof p);
+    } else if constexpr (sizeof(P) == 4) {  // (16-byte pieces lie inside or outside)
+        for (int i = 0; i < n; ++i)
+            if (x + i >= 0 && x + i < w) p |= (uint32_t)row[x + i] << (8 * sizeof(S) * i);
+    }
+    return p;
+}
+
+template <typename S, typename P>
+__global__ __launch_bounds__(kBoxThreads, 4) void transform_box_kernel(const S* __restrict__ src, int w, int h, int d,
+                                                                       S* __restrict__ dst, int tw, int th, int z0,
+                                                                       int nz, Mat12 M, BoxMap B)
+{
+    extern __shared__ __attribute__((aligned(16))) char box[];
+    constexpr unsigned s = kBoxSuper;
+    const unsigned lid = xcd_block(blockIdx.x, gridDim.x), st = lid / (s * s * s), wi = lid % (s * s * s);
+    const unsigned bx = st % B.nsx * s + wi % s, by = st / B.nsx % B.nsy * s + wi / s % s,
+                   bz = st / (B.nsx * B.nsy) * s + wi / (s * s);
+    const int x0 = (int)bx * kT, y0 = (int)by * kT, zb = z0 + (int)bz * kT, ze = z0 + nz;
+    if (bx >= B.nx || by >= B.nby || zb >= ze) return;
+
+    // first texel of the box on each axis (the margin covers the coordinates'
+    // rounding; the host sized the box for it)
+    int org[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        double r = fma(M.m[4 * a], (double)x0, fma(M.m[4 * a + 1], (double)y0, fma(M.m[4 * a + 2], (double)zb, M.m[4 * a + 3])));
+#pragma unroll
+        for (int k = 0; k < 3; ++k) r += fmin(M.m[4 * a + k] * (kT - 1), 0.0);
+        org[a] = __builtin_amdgcn_readfirstlane((int)floor(r - 1e-5));
+    }
+    constexpr int n = sizeof(P) / sizeof(S);
+    if constexpr (sizeof(P) == 16) org[0] &= -n;  // rows are staged from 16-byte boundaries
+
+    // Staging: a thread takes piece q of the rows row, row + step, ... (iy, iz by
+    // counting), four loads in flight; past the last row, and in the threads left
+    // over, it repeats a row.
+    const int rows = B.ny * B.nz, passes = (rows + B.step - 1) / B.step;
+    int row = (int)(threadIdx.x * B.magic_pieces >> 16);
+    const int q = (int)threadIdx.x - row * B.pieces;
+    row = min(row < B.step ? row : 0, rows - 1);
+    int iz = row / B.ny, iy = row - iz * B.ny;
+    uint32_t to = iz * B.plane + iy * B.pitch + q * (int)sizeof(P);
+    const uint32_t to_step = B.step_z * B.plane + B.step_y * B.pitch, to_wrap = B.plane - B.ny * B.pitch;
+    const bool within = org[0] >= 0 && org[0] + B.pieces * n <= w && org[1] >= 0 && org[1] + B.ny <= h && org[2] >= 0 &&
+                        org[2] + B.nz <= d;
+    constexpr int U = 4;
+    if (within) {  // uniform: a box inside the volume needs no checks and 32-bit offsets
+        const char* from = reinterpret_cast<const char*>(src + ((size_t)org[2] * h + org[1]) * w + org[0]);
+        const uint32_t row_bytes = (uint32_t)w * sizeof(S), plane_bytes = row_bytes * (uint32_t)h;
+        const uint32_t step = B.step_z * plane_bytes + B.step_y * row_bytes, wrap = plane_bytes - B.ny * row_bytes;
+        uint32_t off = iz * plane_bytes + iy * row_bytes + q * (uint32_t)sizeof(P);
+        for (int k = 0; k < passes; k += U) {
+            P p[U];
+            uint32_t at[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                at[u] = to;
+                if constexpr (sizeof(P) == 16) p[u] = *reinterpret_cast<const P*>(from + off);
+                else __builtin_memcpy(&p[u], from + off, sizeof(P));
+                if (row + B.step < rows) {
+                    row += B.step;
+                    iy += B.step_y;
+                    const bool over = iy >= B.ny;
+                    off += step + (over ? wrap : 0);
+                    to += to_step + (over ? to_wrap : 0);
+                    iy -= over ? B.ny : 0;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) *reinterpret_cast<P*>(box + at[u]) = p[u];
+        }
+    } else {
+        for (int k = 0; k < passes; ++k) {
+            *reinterpret_cast<P*>(box + to) = load_piece<S, P>(src, w, h, d, org[0] + q * n, org[1] + iy, org[2] + iz);
+            if (row + B.step >= rows) break;
+            row += B.step;
+            iz += B.step_z;
+            iy += B.step_y;
+            to += to_step;
+            if (iy >= B.ny) {
+                iy -= B.ny;
+                ++iz;
+                to += to_wrap;
+            }
+        }
+    }
+    __syncthreads();
+
+    // wavefront: 16 x 4 columns, 8 planes
+    const int x = x0 + (int)(threadIdx.x & 15), y = y0 + (int)(threadIdx.x >> 4 & 15), zw = zb + (int)(threadIdx.x >> 8) * 8;
+    if (x >= tw || y >= th) return;
+    const double xd = (double)x, yd = (double)y, zd = (double)zw;
+    double r[3];  // source coordinates, stepped from plane to plane
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        r[a] = fma(M.m[4 * a + 2], zd, fma(M.m[4 * a], xd, fma(M.m[4 * a + 1], yd, M.m[4 * a + 3])));
+    const double pitch = (double)B.pitch, plane = (double)B.plane;
+    // byte address in LDS of texel (0, 0, 0)
+    const double at0 = (double)lds_address(box) -
+                       fma((double)org[2], plane, fma((double)org[1], pitch, (double)(org[0] * (int)sizeof(S))));
+    S* out = dst + ((size_t)(zw - z0) * th + y) * tw + x;
+    const size_t pstride = (size_t)th * tw;
+    double worst = 0.0;  // largest distance of an unrounded sample from its rounded value
+    auto sample = [&]() -> S {
+        const double fx = floor(r[0]), fy = floor(r[1]), fz = floor(r[2]);
+        const uint32_t shift = (uint32_t)(int)fma(fz, plane, fma(fy, pitch, fma(fx, (double)sizeof(S), at0)));
+        const uint32_t at = shift & ~3u;
+        const double ax = r[0] - fx, ay = r[1] - fy, az = r[2] - fz;
+        const double c0 = lerp(lerp_row<S>(at, shift, ax), lerp_row<S>(at + B.pitch, shift, ax), ay);
+        const double c1 = lerp(lerp_row<S>(at + B.plane, shift, ax), lerp_row<S>(at + B.plane + B.pitch, shift, ax), ay);
+        constexpr double maxv = (double)((1u << (8 * sizeof(S))) - 1u);
+        const double v = lerp(c0, c1, az) * ((maxv + 1.0) / maxv), n = rint(v);  // floor(v + 1/2) off ties
+        worst = fmax(worst, fabs(v - n));
+#pragma unroll
+        for (int a = 0; a < 3; ++a) r[a] += M.m[4 * a + 2];
+        return (S)min((uint32_t)(int)n, (uint32_t)maxv);
+    };
+    if (zw + 8 <= ze) {  // wave-uniform
+#pragma unroll
+        for (int i = 0; i < 8; ++i) out[i * pstride] = sample();
+    } else {
+        for (int i = 0; zw + i < ze; ++i) out[i * pstride] = sample();
+    }
+    if (!(worst < 0.5 - B.guard)) {
+        const double axy[3] = {mul_add(M.m[0], xd, M.m[1], yd), mul_add(M.m[4], xd, M.m[5], yd),
+                               mul_add(M.m[8], xd, M.m[9], yd)};
+        for (int z = zw; z < min(zw + 8, ze); ++z, out += pstride) *out = transform_sample<S>(src, w, h, d, M, axy, z);
+    }
 }
 
 __global__ __launch_bounds__(256) void mask_kernel(float* __restrict__ out, int z, int w, int h, int d,
@@ -198,6 +391,64 @@ static Mat12 to_mat(const float* m)
     return M;
 }
 
+// Bound, in output units, on the difference between the box kernel's
+// arithmetic and the definition over a launch's target voxels: each coordinate is a sum of
+// four terms in either, off by at most 4 roundings of the terms' magnitudes (and 8
+// more from plane to plane);
+// trilinear interpolation changes by at most the sample range per unit of a
+// coordinate, and its own roundings are far below the 1e-9 added.
+static double transform_guard(const Mat12& M, int tw, int th, int zend, double range)
+{
+    double sum = 0.0;
+    for (int a = 0; a < 3; ++a)
+        sum += std::fabs(M.m[4 * a]) * tw + std::fabs(M.m[4 * a + 1]) * th + std::fabs(M.m[4 * a + 2]) * zend +
+               std::fabs(M.m[4 * a + 3]);
+    return (4.0 + 12.0) * 0x1p-53 * sum * range + 1e-9;
+}
+
+// The box kernel where its box fits 64 KiB of LDS, so that one workgroup of a
+// CU computes while another stages, and where the guard leaves few samples to
+// evaluate twice (coordinates up to about 10^7).  Maps that shrink the
+// source by more than about 2 take the general kernel.
+template <typename S, typename P>
+static bool launch_box(const S* src, int w, int h, int d, S* dst, int tw, int th, int z0, int nz, const Mat12& M,
+                       hipStream_t s)
+{
+    BoxMap B;
+    B.guard = transform_guard(M, tw, th, z0 + nz, 65536.0);
+    if (!(B.guard < 1e-3)) return false;
+    int n[3];
+    for (int a = 0; a < 3; ++a) {
+        const double e = (std::fabs(M.m[4 * a]) + std::fabs(M.m[4 * a + 1]) + std::fabs(M.m[4 * a + 2])) * (kT - 1);
+        if (!(e < 140.0)) return false;
+        n[a] = (int)std::ceil(e + 1e-4) + 2;
+    }
+    constexpr int ps = sizeof(P) / sizeof(S);
+    B.pieces = (n[0] + (sizeof(P) == 16 ? 2 * ps - 2 : ps - 1)) / ps;
+    B.ny = n[1];
+    B.nz = n[2];
+    // rows and planes an odd number of pieces apart spread over the banks
+    B.pitch = (B.pieces | 1) * (int)sizeof(P);
+    B.plane = (B.ny | 1) * B.pitch;
+    const size_t lds = (size_t)B.plane * B.nz + 16;  // (a row's last read reaches 8 bytes past it)
+    if (lds > 64 * 1024) return false;
+    B.step = kBoxThreads / B.pieces;
+    B.step_z = B.step / B.ny;
+    B.step_y = B.step % B.ny;
+    B.magic_pieces = (65536u + B.pieces - 1) / B.pieces;
+    B.nx = (unsigned)((tw + kT - 1) / kT);
+    B.nby = (unsigned)((th + kT - 1) / kT);
+    const unsigned nbz = (unsigned)((nz + kT - 1) / kT);
+    B.nsx = (B.nx + kBoxSuper - 1) / kBoxSuper;
+    B.nsy = (B.nby + kBoxSuper - 1) / kBoxSuper;
+    const unsigned long long blocks =
+        (unsigned long long)B.nsx * B.nsy * ((nbz + kBoxSuper - 1) / kBoxSuper) * kBoxSuper * kBoxSuper * kBoxSuper;
+    if (blocks > 0x7fffffffull || (double)w * h * sizeof(S) * B.nz >= 4294967296.0) return false;
+    launch(transform_box_kernel<S, P>, dim3((unsigned)blocks), dim3(kBoxThreads), (unsigned)lds, s, src, w, h, d, dst, tw,
+           th, z0, nz, M, B);
+    return true;
+}
+
 template <typename S>
 static void launch_transform(const S* src, int w, int h, int d, S* dst, int tw, int th, int z0, int nz,
                              const Mat12& M, hipStream_t s)
@@ -209,8 +460,15 @@ static void launch_transform(const S* src, int w, int h, int d, S* dst, int tw, 
     const unsigned long long nblocks = (unsigned long long)nsx * nsy * nsz * kSuper;
     if (nblocks > 0x7fffffffull) throw_msg("transform: target volume too large for one launch");
     TimedScope ts(kTimeTransform, s);
-    launch(transform_kernel<S>, dim3((unsigned)nblocks), dim3(kGX * kGY), 0, s, src, w, h, d, dst, tw, th, z0, nz,
-           M, nbx, nby, nsx, nsy);
+    // 16-byte pieces where every row starts on a 16-byte boundary
+    const bool aligned = (size_t)w * sizeof(S) % 16 == 0 && (uintptr_t)src % 16 == 0;
+    if (aligned ? launch_box<S, uint4>(src, w, h, d, dst, tw, th, z0, nz, M, s)
+                : launch_box<S, uint32_t>(src, w, h, d, dst, tw, th, z0, nz, M, s)) {
+        FMVD_LAUNCH_CHECK();
+        return;
+    }
+    launch(transform_general_kernel<S>, dim3((unsigned)nblocks), dim3(kGX * kGY), 0, s, src, w, h, d, dst, tw, th, z0,
+           nz, M, nbx, nby, nsx, nsy);
     FMVD_LAUNCH_CHECK();
 }
 

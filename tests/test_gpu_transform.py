@@ -114,3 +114,36 @@ def test_transform_global_gather_fallback(fm, orc):
     want = orc.transform(src, M, tshape, bits=16)
     assert (want > 0).mean() > 0.5
     assert np.array_equal(got, want), int(np.count_nonzero(got != want))
+
+
+def rotated(angles, scale, src, dst):
+    """Inverse map about the volume centres: rotations about x, y, z (degrees), then a scale."""
+    a = np.deg2rad(angles)
+    (cx, cy, cz), (sx, sy, sz) = np.cos(a), np.sin(a)
+    A = scale * (np.array([[cz, -sz, 0], [sz, cz, 0], [0, 0, 1]]) @ np.array([[cy, 0, sy], [0, 1, 0], [-sy, 0, cy]])
+                 @ np.array([[1, 0, 0], [0, cx, -sx], [0, sx, cx]]))
+    b = np.array(src[::-1]) / 2 - A @ (np.array(dst[::-1]) / 2)
+    return np.concatenate([A, b[:, None]], 1).astype(np.float32)
+
+
+@pytest.mark.parametrize("bits", [16, 8])
+@pytest.mark.parametrize("shape,tshape,angles,scale", [
+    ((1, 1, 1), (1, 1, 1), (0, 0, 0), 1.0),
+    ((3, 5, 8), (17, 16, 33), (5, -9, 12), 0.9),       # boxes partly and wholly outside the volume
+    ((41, 64, 64), (33, 48, 47), (15, 15, -15), 1.1),  # rows on 16-byte boundaries, boxes inside and across faces
+    ((40, 63, 61), (33, 47, 49), (-15, 10, 15), 1.0),  # odd rows
+    ((30, 50, 66), (30, 50, 66), (45, 45, 45), 1.0),   # a box near the limit of the LDS
+    ((50, 70, 80), (20, 30, 33), (10, 20, 30), 2.4),   # beyond it: the general kernel
+    ((20, 30, 48), (40, 60, 90), (0, 0, 45), 0.4),
+])
+def test_transform_box_edges(fm, orc, bits, shape, tshape, angles, scale):
+    """The boxes a workgroup stages: at the volume's faces, outside it, at both row
+    alignments, at and beyond the size limit."""
+    src = volume(shape, bits, seed=shape[2] + bits) if shape != (1, 1, 1) else np.full(
+        shape, 1 << (bits - 1), np.uint16 if bits == 16 else np.uint8)
+    M = rotated(angles, scale, shape, tshape)
+    dsrc, ddst = to_device(src), empty_device(tshape, src.dtype)
+    fm.transform_device(dsrc.ptr, shape, ddst.ptr, tshape, M, bits=bits)
+    fm.device_synchronize()
+    want = orc.transform(src.astype(np.uint16), M, tshape, bits=bits).astype(src.dtype)
+    assert np.array_equal(from_device(ddst, src.dtype), want)
