@@ -323,8 +323,8 @@ template <int... Rs> struct RadixList {
     }
 };
 
-// G_ (optional): rows per workgroup of the row kernels, sequences per
-// workgroup of the column kernel (0 = their default).
+// G_ (optional): rows per workgroup of the row kernels (0 = their default).
+// C_ (optional): columns per workgroup of the column kernel (0 = its default).
 // W_ (optional): minimum resident waves per SIMD the kernels are compiled for
 // (amdgpu_waves_per_eu; 1 = whatever the workgroup size implies); a higher
 // value caps the VGPRs per thread so that more workgroups fit on a CU.
@@ -332,10 +332,11 @@ template <int... Rs> struct RadixList {
 // then the imaginary parts, through a float buffer (E = float) instead of
 // moving complex values through a float2 buffer (E = float2): half the LDS per
 // sequence, for twice the synchronisations.
-template <int N_, int T_, typename Radices, int G_ = 0, int W_ = 1, bool S_ = false> struct PlanDef {
+template <int N_, int T_, typename Radices, int G_ = 0, int W_ = 1, bool S_ = false, int C_ = 0> struct PlanDef {
     static constexpr int N = N_;
     static constexpr int T = T_;
     static constexpr int G = G_;
+    static constexpr int COLS = C_;
     static constexpr int WPE = W_;
     static constexpr int P = N_ / T_;
     static constexpr bool SPLIT = S_;
@@ -344,21 +345,25 @@ template <int N_, int T_, typename Radices, int G_ = 0, int W_ = 1, bool S_ = fa
     static constexpr int NP = Radices::count;
 };
 
-// Default plans.  Constraint: every radix divides P.
+// Default plans.  Constraint: every radix divides P.  The columns per workgroup are the
+// fewest that keep a wavefront full: a smaller group waits for fewer wavefronts at its
+// barriers and ends sooner (us a launch with 256 threads, then with one wavefront: 512 x
+// 64 planes of 512 27.3, 24.8; 1024 x 32 of 1024 30.6, 28.9; 1536 x 8 of 1536 34.7, 33.8).
+// Rows of 128 take 8 a workgroup where 16 left half of the CUs without work on one plane.
 template <int N> struct Plan;
 template <> struct Plan<8> : PlanDef<8, 1, RadixList<8>> {};
 template <> struct Plan<16> : PlanDef<16, 1, RadixList<16>> {};
 template <> struct Plan<32> : PlanDef<32, 2, RadixList<16, 2>> {};
 template <> struct Plan<64> : PlanDef<64, 4, RadixList<16, 4>> {};
-template <> struct Plan<128> : PlanDef<128, 8, RadixList<16, 8>> {};
-template <> struct Plan<256> : PlanDef<256, 16, RadixList<16, 16>> {};
-template <> struct Plan<512> : PlanDef<512, 32, RadixList<16, 16, 2>> {};
+template <> struct Plan<128> : PlanDef<128, 8, RadixList<16, 8>, 8> {};
+template <> struct Plan<256> : PlanDef<256, 16, RadixList<16, 16>, 16, 1, false, 4> {};
+template <> struct Plan<512> : PlanDef<512, 32, RadixList<16, 16, 2>, 8, 1, false, 2> {};
 template <> struct Plan<768> : PlanDef<768, 64, RadixList<4, 4, 4, 12>, 8, 4> {};
-template <> struct Plan<1024> : PlanDef<1024, 64, RadixList<16, 16, 4>> {};
+template <> struct Plan<1024> : PlanDef<1024, 64, RadixList<16, 16, 4>, 8, 1, false, 1> {};
 template <> struct Plan<1280> : PlanDef<1280, 64, RadixList<4, 4, 4, 20>, 8, 4, true> {};
-template <> struct Plan<1536> : PlanDef<1536, 64, RadixList<8, 8, 24>> {};
+template <> struct Plan<1536> : PlanDef<1536, 64, RadixList<8, 8, 24>, 8, 1, false, 1> {};
 template <> struct Plan<1792> : PlanDef<1792, 64, RadixList<4, 4, 4, 28>> {};
-template <> struct Plan<2048> : PlanDef<2048, 128, RadixList<16, 16, 8>> {};
+template <> struct Plan<2048> : PlanDef<2048, 128, RadixList<16, 16, 8>, 8, 1, false, 1> {};
 template <> struct Plan<2560> : PlanDef<2560, 64, RadixList<8, 8, 8, 5>> {};
 template <> struct Plan<3072> : PlanDef<3072, 64, RadixList<16, 16, 12>> {};
 template <> struct Plan<3584> : PlanDef<3584, 64, RadixList<8, 8, 8, 7>> {};
@@ -379,42 +384,38 @@ template <> struct Plan<7168> : PlanDef<7168, 256, RadixList<4, 4, 4, 4, 4, 7>> 
 template <> struct Plan<7680> : PlanDef<7680, 128, RadixList<4, 4, 4, 4, 2, 15>> {};
 template <> struct Plan<8192> : PlanDef<8192, 256, RadixList<16, 16, 32>> {};
 
-// Alternative plans for the extents of the benchmark workloads, selected at
-// run time per kernel kind (fewer registers per thread at the price of more
-// LDS exchanges, or the reverse).  PlanV<N, 0> is Plan<N>.
+// Alternative plans, selected at run time per kernel kind (fewer registers
+// per thread at the price of more LDS exchanges, or the reverse; rows or columns per
+// workgroup).  PlanV<N, 0> is Plan<N>; default_variants names an untuned plan's.
 constexpr int kPlanVariants = 3;
 template <int N, int V> struct PlanV : Plan<N> {
     static constexpr bool distinct = (V == 0);
     static constexpr int variant = 0;
 };
-#define FMVD_PLAN_VARIANT_GWS(n, v, t, g, w, s, ...)                                  \
-    template <> struct PlanV<n, v> : PlanDef<n, t, RadixList<__VA_ARGS__>, g, w, s> {  \
-        static constexpr bool distinct = true;                                        \
-        static constexpr int variant = v;                                             \
+#define FMVD_PLAN_VARIANT(n, v, t, g, c, w, s, ...)                                       \
+    template <> struct PlanV<n, v> : PlanDef<n, t, RadixList<__VA_ARGS__>, g, w, s, c> {  \
+        static constexpr bool distinct = true;                                           \
+        static constexpr int variant = v;                                                \
     };
-#define FMVD_PLAN_VARIANT_GW(n, v, t, g, w, ...) FMVD_PLAN_VARIANT_GWS(n, v, t, g, w, false, __VA_ARGS__)
-#define FMVD_PLAN_VARIANT_G(n, v, t, g, ...) FMVD_PLAN_VARIANT_GW(n, v, t, g, 1, __VA_ARGS__)
-#define FMVD_PLAN_VARIANT(n, v, t, ...) FMVD_PLAN_VARIANT_G(n, v, t, 0, __VA_ARGS__)
-FMVD_PLAN_VARIANT(256, 1, 32, 8, 8, 4)
-FMVD_PLAN_VARIANT(512, 1, 64, 8, 8, 8)
-FMVD_PLAN_VARIANT_GW(768, 1, 64, 4, 5, 4, 4, 4, 12)
-FMVD_PLAN_VARIANT_GW(768, 2, 64, 4, 6, 4, 4, 4, 12)
-FMVD_PLAN_VARIANT(1024, 1, 64, 8, 8, 16)
-FMVD_PLAN_VARIANT(1024, 2, 128, 8, 8, 4, 4)
-FMVD_PLAN_VARIANT_GW(1280, 1, 64, 4, 4, 4, 4, 4, 20)
-// variant 1 with split exchanges: 22 KB of LDS per 4-row workgroup, so four
-// workgroups (4 waves per SIMD) fit where variant 1's 44 KB allow three
-FMVD_PLAN_VARIANT_GWS(1280, 2, 64, 4, 4, true, 4, 4, 4, 20)
-FMVD_PLAN_VARIANT(1536, 1, 64, 8, 8, 8, 3)
-FMVD_PLAN_VARIANT(1536, 2, 128, 4, 4, 4, 4, 6)
+//                N  v   T  G  C  W  split  radices
+FMVD_PLAN_VARIANT(128, 1, 16, 8, 8, 1, false, 8, 4, 4)
+FMVD_PLAN_VARIANT(256, 1, 32, 16, 8, 1, false, 8, 4, 8)
+FMVD_PLAN_VARIANT(512, 1, 64, 8, 1, 6, false, 8, 8, 8)
+FMVD_PLAN_VARIANT(768, 1, 64, 4, 0, 5, false, 4, 4, 4, 12)
+FMVD_PLAN_VARIANT(768, 2, 64, 4, 0, 6, false, 4, 4, 4, 12)
+FMVD_PLAN_VARIANT(1024, 1, 64, 8, 1, 1, false, 8, 8, 16)
+FMVD_PLAN_VARIANT(1024, 2, 128, 8, 1, 1, false, 8, 4, 4, 8)
+FMVD_PLAN_VARIANT(1280, 1, 64, 4, 0, 4, false, 4, 4, 4, 20)
+// variant 1 with split exchanges: 24 KB of LDS per 4-row workgroup, so four
+// workgroups (4 waves per SIMD) fit where variant 1's 45 KB allow three
+FMVD_PLAN_VARIANT(1280, 2, 64, 4, 0, 4, true, 4, 4, 4, 20)
+FMVD_PLAN_VARIANT(1536, 1, 64, 0, 1, 1, false, 8, 8, 8, 3)
+FMVD_PLAN_VARIANT(1536, 2, 128, 4, 0, 1, false, 4, 4, 4, 4, 6)
 // one 2-wavefront sequence per column workgroup (22 KB of LDS, 4 waves per
 // SIMD), radix 20 last: 12 % faster than variant 2 on the 2560-point columns
-FMVD_PLAN_VARIANT_GW(2560, 1, 128, 1, 4, 2, 4, 4, 4, 20)
-FMVD_PLAN_VARIANT(2560, 2, 128, 4, 4, 4, 4, 10)
+FMVD_PLAN_VARIANT(2560, 1, 128, 1, 1, 4, false, 2, 4, 4, 4, 20)
+FMVD_PLAN_VARIANT(2560, 2, 128, 0, 2, 1, false, 4, 4, 4, 4, 10)
 #undef FMVD_PLAN_VARIANT
-#undef FMVD_PLAN_VARIANT_G
-#undef FMVD_PLAN_VARIANT_GW
-#undef FMVD_PLAN_VARIANT_GWS
 
 // A plan is valid when its radices multiply to N and each divides P.
 template <typename PL> constexpr bool plan_valid()

@@ -70,8 +70,8 @@ __global__ __launch_bounds__(RowCfg<PL>::THREADS, PL::WPE) void batch_update_ker
     const int lid = (int)xcd_remap(blockIdx.x, gridDim.x);
     const int e = find_entry(list, n, lid);
     const BatchSeg& S = segs[list[e]];
-    const int local = lid - list[n + e], nrg = g.H / C::G;
-    const int rg = local % nrg, pl = local / nrg;
+    int rg, pl;
+    grouped_tile((unsigned)(lid - list[n + e]), g.H / C::G, S.nplanes, rg, pl);
     const long p = S.plane0 + pl;
     update_tile<PL>(seg_geom(g, S), XE + p * xstride, XT + p * xstride, ES + p * estride, S.w[view], rg * C::G,
                     lds);
@@ -88,9 +88,8 @@ __global__ __launch_bounds__(ColCfg<PL>::THREADS, PL::WPE) void batch_col_kernel
     const int lid = (int)xcd_remap(blockIdx.x, gridDim.x);
     const int e = find_entry(list, n, lid);
     const BatchSeg& S = segs[list[e]];
-    const int local = lid - list[n + e];
-    // plane-fastest inside a volume: consecutive blocks reuse the kernel rows
-    const int pl = local % S.nplanes, grp = local / S.nplanes;
+    int pl, grp;
+    column_tile<C::SQ>((unsigned)(lid - list[n + e]), S.nplanes, grp, pl);
     const long p = S.plane0 + pl;
     col_tile<PL>(g, Xin + p * xstride, Xout + p * xstride, hat ? S.Kh[view] : S.K[view], grp, lds,
                  hat && S.khconj ? -1.0f : 1.0f);

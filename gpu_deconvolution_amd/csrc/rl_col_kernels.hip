@@ -33,19 +33,7 @@ __global__ __launch_bounds__(ColCfg<PL>::THREADS, PL::WPE) void col_conv_kernel(
     __shared__ typename C::E lds[C::SQ * C::L];
     const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
     int p, grp;
-    if constexpr (C::SQ == 1) {
-        // one column per workgroup: the two columns of a kx pair, which share
-        // every 16-byte word of the spectrum, run back to back so that their
-        // half-word writes meet in L2; then the planes, so that consecutive
-        // pairs of blocks reuse the same kernel columns (N is even)
-        const unsigned q = lid >> 1;
-        p = (int)(q % (unsigned)nplanes);
-        grp = (int)((q / (unsigned)nplanes) * 2u + (lid & 1u));
-    } else {
-        // plane-fastest: consecutive logical blocks reuse the same kernel rows
-        p = (int)(lid % (unsigned)nplanes);
-        grp = (int)(lid / (unsigned)nplanes);
-    }
+    column_tile<C::SQ>(lid, nplanes, grp, p);
     col_tile<PL>(g, Xin + p * xstride, Xout + p * xstride, K, grp, lds, ksign);
 }
 

@@ -333,13 +333,14 @@ template <typename S> struct Plan {
     // fastest.  times[kind*3 + variant] receives the mean launch time in ms
     // (negative where the variant does not exist).
     // Key of this plan's tuning in the autotuner cache file: device, extents,
-    // sample type, kernel-hat form and the planes the launches cover.
+    // sample type, kernel-hat form, the planes the launches cover and the plan
+    // list's version (entries of another list are not taken).
     std::string tune_key(int planes) const
     {
         hipDeviceProp_t prop;
         FMVD_HIP(hipGetDeviceProperties(&prop, device));
         char key[256];
-        snprintf(key, sizeof key, "%s|%d|%dx%d|u%d|c%d|p%d", prop.gcnArchName, cus, fftH, fftW, (int)(8 * sizeof(S)),
+        snprintf(key, sizeof key, "%s|%d|%dx%d|u%d|c%d|l2|p%d", prop.gcnArchName, cus, fftH, fftW, (int)(8 * sizeof(S)),
                  khatConj ? 1 : 0, planes);
         for (char* c = key; *c; ++c)
             if (*c == ' ') *c = '_';

@@ -36,21 +36,6 @@ __global__ __launch_bounds__(RowCfg<PL>::THREADS, PL::WPE) void row_ratio_kernel
 }
 
 // ------------------------------------------------------------------ pass D
-// Row group / plane of a block when planes are taken in groups of kPlaneGroup
-// with the plane fastest inside a group: the blocks that run together on one
-// XCD then share the weight rows in its L2, while a row group's neighbours
-// (which share the tile's cache lines) stay only kPlaneGroup blocks away.
-constexpr int kPlaneGroup = 8;
-__device__ __forceinline__ void grouped_tile(unsigned lid, int nrg, int nplanes, int& rg, int& p)
-{
-    const int pg = (int)(lid / (unsigned)(nrg * kPlaneGroup));
-    const int base = pg * kPlaneGroup;
-    const int kk = min(kPlaneGroup, nplanes - base);
-    const int rem = (int)lid - pg * nrg * kPlaneGroup;
-    rg = rem / kk;
-    p = base + rem % kk;
-}
-
 template <typename PL>
 __global__ __launch_bounds__(RowCfg<PL>::THREADS, PL::WPE) void row_update_kernel(
     RowGeom g, float2* XE, const float2* XC, float* __restrict__ ES, long xstride,

@@ -33,6 +33,37 @@ __device__ __forceinline__ unsigned xcd_remap(unsigned bid, unsigned nblocks)
     return x * q + (x < rem ? x : rem) + k;
 }
 
+// Row group / plane of a block when planes are taken in groups of kPlaneGroup
+// with the plane fastest inside a group: the blocks that run together on one
+// XCD then share the weight rows in its L2, while a row group's neighbours
+// (which share the tile's cache lines) stay only kPlaneGroup blocks away.
+constexpr int kPlaneGroup = 8;
+__device__ __forceinline__ void grouped_tile(unsigned lid, int nrg, int nplanes, int& rg, int& p)
+{
+    const int pg = (int)(lid / (unsigned)(nrg * kPlaneGroup));
+    const int base = pg * kPlaneGroup;
+    const int kk = min(kPlaneGroup, nplanes - base);
+    const int rem = (int)lid - pg * nrg * kPlaneGroup;
+    rg = rem / kk;
+    p = base + rem % kk;
+}
+
+// Column group / plane of a block, plane-fastest: consecutive blocks reuse the
+// same kernel columns.  With one column per workgroup the two columns of a kx
+// pair, which share every 16-byte word of the spectrum, run back to back so that
+// their half-word writes meet in L2 (the column count is even).
+template <int SQ> __device__ __forceinline__ void column_tile(unsigned lid, int nplanes, int& grp, int& p)
+{
+    if constexpr (SQ == 1) {
+        const unsigned q = lid >> 1;
+        p = (int)(q % (unsigned)nplanes);
+        grp = (int)((q / (unsigned)nplanes) * 2u + (lid & 1u));
+    } else {
+        p = (int)(lid % (unsigned)nplanes);
+        grp = (int)(lid / (unsigned)nplanes);
+    }
+}
+
 // LDS row pitch >= len with L = 16/G (mod 16).  The LDS serves 8-byte
 // accesses a quarter-wavefront (16 lanes, 32 four-byte banks) per cycle; in
 // the transposed tile access those lanes hold G consecutive rows times 16/G
@@ -85,20 +116,22 @@ template <typename PL_> struct RowCfg {
     static constexpr int RLI = last_radix<PL, +1>();   // layout on exit of the inverse (= forward entry)
     static constexpr int RLF = last_radix<PL, -1>();   // layout on exit of the forward
     static_assert(RLI == first_radix<PL, -1>(), "inverse exit layout must match forward entry");
+    // whether a tile's accesses share one address register (see lds_pad below)
+    static constexpr bool AFFINE_T = N % 16 == 0 && (T % 16 == 0 || T == 8);
+    static constexpr bool AFFINE_I = AFFINE_T && (N / RFI) % 16 == 0, AFFINE_F = AFFINE_T && (N / RLF) % 16 == 0;
 };
 
-// LDS addressing.  lds_pad(base + c) = lds_pad(base) + c + c/16 whenever c is a
-// multiple of 16, and lds_pad(A - t) = A + A/16 + lds_mirror(t) whenever A is;
-// the affine forms let every access of a thread share one address register
-// and use immediate offsets.
+// LDS addressing.  With t below T and c a multiple of T, lds_pad(t + c) = lds_pad(t) + c + c/16
+// where T is a multiple of 16 (so is c), and where T is 8 (t + c crosses no multiple
+// of 16 that c does not); likewise lds_pad(A - t) for a multiple A of T is A + A/16 +
+// lds_mirror(t) when A is a multiple of 16, and A + A/16 - t when it is not.
+// The affine forms let every access of a thread share one address register and
+// use immediate offsets.
 __device__ __forceinline__ int lds_mirror(int t) { return -t + ((-t) >> 4); }
-template <int C> constexpr int pad_c() { return C + C / 16; }
-
-// The affine forms apply when the sequence's thread count and every slot
-// offset of the given register layout are multiples of 16.
-template <typename C, int R> constexpr bool affine_layout()
+constexpr int pad_c(int c) { return c + c / 16; }
+template <int A> __device__ __forceinline__ int lds_mirrored(int t, int mirror_t)
 {
-    return C::T % 16 == 0 && (C::N / R) % 16 == 0 && C::N % 16 == 0;
+    return pad_c(A) + (A % 16 == 0 ? mirror_t : -t);
 }
 
 // Tile element k of thread tid (q = tid + k * THREADS) in the spectrum
@@ -137,14 +170,14 @@ __device__ __forceinline__ void fetch_tile(float2* pre, const float2* __restrict
 template <typename C, int COMP = 0>
 __device__ __forceinline__ void stage_tile(typename Comp<COMP>::E* lds, const float2* pre, int tid)
 {
-    if constexpr (C::T % 16 == 0) {
+    if constexpr (C::AFFINE_T) {
         int g, kx0;
         tile_elem<C>(tid, 0, g, kx0);
         typename Comp<COMP>::E* dst = lds + g * C::L + lds_pad(kx0);
 #pragma unroll
         for (int k = 0; k < C::P; ++k) {
             float2 x = pre[k];
-            dst[k * pad_c<C::T>()] = Comp<COMP>::of(x);
+            dst[pad_c(k * C::T)] = Comp<COMP>::of(x);
         }
     } else {
 #pragma unroll
@@ -171,18 +204,20 @@ __device__ __forceinline__ float2 c2r_combine(float2 xk, float2 xmc, float2 w)
 
 // exp(-2 pi i (p + c) / W) for a compile-time c, from w0 = exp(-2 pi i p / W)
 // (one load per thread) times the constant exp(-2 pi i c / W): the tables'
-// loads, not their arithmetic, bound the row passes.
-template <int N, int c> __device__ __forceinline__ float2 twiddle_w(float2 w0)
+// loads, not their arithmetic, bound the row passes.  Rows of 8 threads read the
+// table, w = exp(-2 pi i p / W), as the rows of fewer do.
+template <typename C, int c> __device__ __forceinline__ float2 twiddle_w(float2 w0, const float2* w)
 {
-    if constexpr (c == 0) return w0;
-    else return cmul(w0, ct_tw<-1, (long)c, 2L * N>());
+    if constexpr (C::T < 16) return w[c];
+    else if constexpr (c == 0) return w0;
+    else return cmul(w0, ct_tw<-1, (long)c, 2L * C::N>());
 }
 
 template <typename C>
-__device__ __forceinline__ void c2r_pre(float2* v, const float2* row, int t, const float2* __restrict__ twW)
+__device__ __forceinline__ void c2r_pre(float2* v, const float2* row, int t, const float2* twW)
 {
     using PL = typename C::PL;
-    if constexpr (affine_layout<C, C::RFI>()) {
+    if constexpr (C::AFFINE_I) {
         const int pt = lds_pad(t), mt = lds_mirror(t);
         const float2 w0 = twW[t];
         static_for<0, C::P>([&]<int i>() {
@@ -191,10 +226,10 @@ __device__ __forceinline__ void c2r_pre(float2* v, const float2* row, int t, con
             const float2 xk = row[pt + c + c / 16];
             if constexpr (i == 0) {
                 const int im = t == 0 ? pt : C::N + C::N / 16 + mt;
-                const float2 z = c2r_combine(xk, row[im], w0);
+                const float2 z = c2r_combine(xk, row[im], twiddle_w<C, 0>(w0, twW + t));
                 v[i] = t == 0 ? make_float2(xk.x + xk.y, xk.x - xk.y) : z;
             } else {
-                v[i] = c2r_combine(xk, row[(C::N - c) + (C::N - c) / 16 + mt], twiddle_w<C::N, c>(w0));
+                v[i] = c2r_combine(xk, row[lds_mirrored<C::N - c>(t, mt)], twiddle_w<C, c>(w0, twW + t));
             }
         });
     } else {
@@ -214,10 +249,9 @@ __device__ __forceinline__ void c2r_pre(float2* v, const float2* row, int t, con
 // and d.x = re X[p] - re X[N-p]; after the imaginary parts, a.y and d.y; then
 // Z'[p] = (a.x - b.y, a.y + b.x), b = d * conj(w).
 template <typename C>
-__device__ __forceinline__ void stage_c2r_pre_split(float2* v, float* lds, int tid, int seq, int t,
-                                                    const float2* __restrict__ twW)
+__device__ __forceinline__ void stage_c2r_pre_split(float2* v, float* lds, int tid, int seq, int t, const float2* twW)
 {
-    static_assert(affine_layout<C, C::RFI>() && C::T % 16 == 0, "split exchanges need the affine layout");
+    static_assert(C::AFFINE_I && C::T % 16 == 0, "split exchanges need the affine layout");
     constexpr int M = C::N / C::RFI;
     const float* row = lds + seq * C::L;
     const int pt = lds_pad(t), mt = lds_mirror(t);
@@ -241,7 +275,7 @@ __device__ __forceinline__ void stage_c2r_pre_split(float2* v, float* lds, int t
         constexpr int c = (i / C::RFI) * C::T + (i % C::RFI) * M;
         const float yk = row[pt + c + c / 16];
         const float ym = i == 0 ? row[t == 0 ? pt : C::N + C::N / 16 + mt] : row[(C::N - c) + (C::N - c) / 16 + mt];
-        const float2 b = cmulc(make_float2(dx[i], yk + ym), twiddle_w<C::N, c>(w0));
+        const float2 b = cmulc(make_float2(dx[i], yk + ym), twiddle_w<C, c>(w0, twW + t));
         const float2 z = make_float2(ax[i] - b.y, (yk - ym) + b.x);
         v[i] = (i == 0 && t == 0) ? make_float2(x0 + yk, x0 - yk) : z;
     });
@@ -264,10 +298,9 @@ __device__ __forceinline__ float2 r2c_combine(float2 zk, float2 zmc, float2 w, f
 // (s = Z[k] + conj Z[N-k] and d = Z[k] - conj Z[N-k] by parts).
 template <typename C>
 __device__ __forceinline__ void r2c_post_store_split(float2* v, float* lds, float2* __restrict__ X, int H, int y0,
-                                                     int tid, int seq, int t, const float2* __restrict__ twW,
-                                                     float scale)
+                                                     int tid, int seq, int t, const float2* twW, float scale)
 {
-    static_assert(affine_layout<C, C::RLF>() && C::T % 16 == 0, "split exchanges need the affine layout");
+    static_assert(C::AFFINE_F && C::T % 16 == 0, "split exchanges need the affine layout");
     constexpr int M = C::N / C::RLF;
     const float h = 0.5f * scale;
     float* dst = lds + seq * C::L + lds_pad(t);
@@ -306,15 +339,14 @@ __device__ __forceinline__ void r2c_post_store_split(float2* v, float* lds, floa
         const float zm = k == 0 ? r[kx0 == 0 ? pk : C::N + C::N / 16 + mk] : r[(C::N - c) + (C::N - c) / 16 + mk];
         const float2 fe = make_float2(sx[k] * h, (zk - zm) * h);
         const float2 fo = make_float2(h * (zk + zm), -h * dx[k]);
-        const float2 z = cadd(fe, cmul(twiddle_w<C::N, c>(w0), fo));
+        const float2 z = cadd(fe, cmul(twiddle_w<C, c>(w0, twW + kx0), fo));
         X[off0 + k * step] = (k == 0 && kx0 == 0) ? make_float2((z0 + zk) * scale, (z0 - zk) * scale) : z;
     });
 }
 
 template <typename C>
 __device__ __forceinline__ void r2c_post_store(float2* v, typename C::E* lds, float2* __restrict__ X, int H,
-                                               int y0, int tid, int seq, int t, const float2* __restrict__ twW,
-                                               float scale)
+                                               int y0, int tid, int seq, int t, const float2* twW, float scale)
 {
     if constexpr (C::PL::SPLIT) {
         r2c_post_store_split<C>(v, lds, X, H, y0, tid, seq, t, twW, scale);
@@ -323,7 +355,7 @@ __device__ __forceinline__ void r2c_post_store(float2* v, typename C::E* lds, fl
     using PL = typename C::PL;
     const float h = 0.5f * scale;
     float2* row = lds + seq * C::L;
-    if constexpr (affine_layout<C, C::RLF>()) {
+    if constexpr (C::AFFINE_F) {
         constexpr int M = C::N / C::RLF;
         float2* dst = row + lds_pad(t);
 #pragma unroll
@@ -336,7 +368,7 @@ __device__ __forceinline__ void r2c_post_store(float2* v, typename C::E* lds, fl
         for (int i = 0; i < C::P; ++i) row[lds_pad(slot_pos<PL, C::RLF>(t, i))] = v[i];
     }
     __syncthreads();
-    if constexpr (C::T % 16 == 0) {
+    if constexpr (C::AFFINE_T) {
         int g, kx0;
         tile_elem<C>(fresh(tid), 0, g, kx0);
         const float2* r = lds + g * C::L;
@@ -349,10 +381,10 @@ __device__ __forceinline__ void r2c_post_store(float2* v, typename C::E* lds, fl
             float2 xo;
             if constexpr (k == 0) {
                 const int im = kx0 == 0 ? pk : C::N + C::N / 16 + mk;
-                const float2 z = r2c_combine(zk, r[im], w0, h);
+                const float2 z = r2c_combine(zk, r[im], twiddle_w<C, 0>(w0, twW + kx0), h);
                 xo = kx0 == 0 ? make_float2((zk.x + zk.y) * scale, (zk.x - zk.y) * scale) : z;
             } else {
-                xo = r2c_combine(zk, r[(C::N - c) + (C::N - c) / 16 + mk], twiddle_w<C::N, c>(w0), h);
+                xo = r2c_combine(zk, r[lds_mirrored<C::N - c>(kx0, mk)], twiddle_w<C, c>(w0, twW + kx0), h);
             }
             X[off0 + k * step] = xo;
         });
@@ -438,8 +470,8 @@ __device__ __forceinline__ void row_c2r(float2* v, typename C::E* lds, int tid, 
 
 // ------------------------------------------------------------- row tiles
 // Each works on the G rows [y0, y0+G) of one padded plane; lds holds
-// G*RowCfg::L complex.  g carries the FFT extent (uniform over the launch)
-// and the data extent and pad half-widths of the plane's volume.
+// G*RowCfg::L elements.  g carries the FFT extent (uniform over the launch) and the data
+// extent and pad half-widths of the plane's volume.
 
 // Pass B: X <- R2C(Q > 1 ? D / Q : Q) * scale, Q = C2R(X).  divide_kernel_{16,8},
 // fmvd_deconvolve_cuda.impl.cu:159-176; the data is read unpadded through the
@@ -447,8 +479,7 @@ __device__ __forceinline__ void row_c2r(float2* v, typename C::E* lds, int tid, 
 // is 1, or 1/W when pass C's kernel spectrum is pass A's (which carries 1/H only).
 template <typename SAMPLE, typename PL>
 __device__ __forceinline__ void ratio_tile(const RowGeom& g, float2* __restrict__ Xp,
-                                           const SAMPLE* __restrict__ dplane, int y0, typename PL::E* lds,
-                                           float scale)
+                                           const SAMPLE* __restrict__ dplane, int y0, typename PL::E* lds, float scale)
 {
     using C = RowCfg<PL>;
     using PairT = typename PairOf<SAMPLE>::type;
@@ -480,7 +511,7 @@ __device__ __forceinline__ void ratio_tile(const RowGeom& g, float2* __restrict_
         v[i].x = q0 > 1.0f ? d0 * __builtin_amdgcn_rcpf(q0) : q0;
         v[i].y = q1 > 1.0f ? d1 * __builtin_amdgcn_rcpf(q1) : q1;
     }
-    fft_regs<PL, -1>(v, row, t, g.twP[PL::variant]);
+    fft_regs<PL, -1>(v, row, t, g.twP[C::PL::variant]);
     r2c_post_store<C>(v, lds, Xp, g.H, y0, tid, seq, t, g.twW, scale);
 }
 
@@ -519,7 +550,7 @@ __device__ __forceinline__ void update_tile(const RowGeom& g, float2* XEp,
         v[i].y = e.y + c1;
         erow[t + c] = v[i];
     }
-    fft_regs<PL, -1>(v, row, t, g.twP[PL::variant]);
+    fft_regs<PL, -1>(v, row, t, g.twP[C::PL::variant]);
     r2c_post_store<C>(v, lds, XEp, g.H, y0, tid, seq, t, g.twW, 1.0f / (float)g.W);
 }
 
@@ -542,7 +573,7 @@ __device__ __forceinline__ void init_tile(const RowGeom& g, float2* __restrict__
         v[i].y = erow[pad_index(2 * n + 1, g.dataW, g.dkX)];
         esrow[n] = v[i];
     }
-    fft_regs<PL, -1>(v, row, t, g.twP[PL::variant]);
+    fft_regs<PL, -1>(v, row, t, g.twP[C::PL::variant]);
     r2c_post_store<C>(v, lds, XEp, g.H, y0, tid, seq, t, g.twW, 1.0f / (float)g.W);
 }
 
@@ -570,7 +601,7 @@ template <typename PL_> struct ColCfg {
     static constexpr int SQ0 = (256 / T) < 1 ? 1 : (256 / T);
     static constexpr int SQ1 = SQ0 > 16 ? 16 : SQ0;
     static constexpr int SQ2 = 65536 / (L * (int)sizeof(E)) < 1 ? 1 : 65536 / (L * (int)sizeof(E));
-    static constexpr int SQ = PL::G ? PL::G : pow2_floor(SQ1 < SQ2 ? SQ1 : SQ2);
+    static constexpr int SQ = PL::COLS ? PL::COLS : pow2_floor(SQ1 < SQ2 ? SQ1 : SQ2);
     static constexpr int THREADS = SQ * T;
     static constexpr int RF = first_radix<PL, -1>();
     static constexpr int RL = last_radix<PL, -1>();
@@ -578,18 +609,23 @@ template <typename PL_> struct ColCfg {
     static_assert(RF == last_radix<PL, +1>(), "inverse exit layout must match forward entry");
 };
 
-// v[i] *= Kr[y] at the inverse-entry positions y of thread t, with Kr[y]'s
-// imaginary part times ksign (-1: the conjugate); Kr is one kx column of a
-// kernel spectrum (contiguous along y).  The sign is a multiply, not a second
-// code path, so every kernel that inlines this computes the same bits.
-template <typename PL>
-__device__ __forceinline__ void col_kmul(float2* v, const float2* __restrict__ Kr, int t, float ksign)
+// k[i] = Kr[y] at the inverse-entry positions y of thread t; Kr is one kx column
+// of a kernel spectrum (contiguous along y).
+template <typename PL> __device__ __forceinline__ void col_kload(float2* k, const float2* __restrict__ Kr, int t)
 {
-    constexpr int RL = last_radix<PL, -1>();
+#pragma unroll
+    for (int i = 0; i < PL::P; ++i) k[i] = Kr[slot_pos<PL, last_radix<PL, -1>()>(t, i)];
+}
+// v[i] *= Kr[y], loaded beforehand (EARLY, in k) or here, with its imaginary part
+// times ksign (-1: the conjugate).  The sign is a multiply, not a second code path, so
+// every kernel that inlines this computes the same bits.
+template <typename PL, bool EARLY>
+__device__ __forceinline__ void col_kmul(float2* v, const float2* k, const float2* __restrict__ Kr, int t, float ksign)
+{
 #pragma unroll
     for (int i = 0; i < PL::P; ++i) {
-        const float2 k = Kr[slot_pos<PL, RL>(t, i)];
-        v[i] = cmul(v[i], make_float2(k.x, ksign * k.y));
+        const float2 x = EARLY ? k[i] : Kr[slot_pos<PL, last_radix<PL, -1>()>(t, i)];
+        v[i] = cmul(v[i], make_float2(x.x, ksign * x.y));
     }
 }
 
@@ -624,6 +660,15 @@ __device__ __forceinline__ void col_tile(const ColGeom& g, const float2* Xin, fl
     float2 v[C::P];
 #pragma unroll
     for (int i = 0; i < C::P; ++i) v[i] = xin[2 * slot_pos<PL, C::RF>(t, i)];
+    // The kernel column loads behind the data, ahead of the FFT, where that costs no resident
+    // wavefront: us per launch over 16.8 M pixels at lengths 512, 1024, 2048 (16 values
+    // per thread): 25.9 -> 24.3, 27.6 -> 25.8, 30.4 -> 29.1; with 20 (2560, 105 M pixels)
+    // 219 -> 251.  Shorter columns (256: 24.0 -> 22.5) load it where they use it: there
+    // the order changes which product of a sum is fused, and so the results' last bits.
+    constexpr bool EARLY_K = C::P <= 16 && C::H >= 512;
+    const float2* Kr = K + (unsigned)(kx * H);
+    float2 kr[EARLY_K ? C::P : 1];
+    if constexpr (EARLY_K) col_kload<PL>(kr, Kr, t);
     fft_regs<PL, -1>(v, row, t, g.twP[PL::variant]);
 
     if (grp == 0) {  // workgroup-uniform: this group holds the packed DC/Nyquist sequence
@@ -633,7 +678,6 @@ __device__ __forceinline__ void col_tile(const ColGeom& g, const float2* Xin, fl
         }
         seq_sync<PL>();
         if (seq == 0) {
-            const float2* K0 = K;                         // kx = 0
             const float2* KN = K + (unsigned)(g.N * H);  // kx = N, contiguous
 #pragma unroll
             for (int i = 0; i < C::P; ++i) {
@@ -643,17 +687,17 @@ __device__ __forceinline__ void col_tile(const ColGeom& g, const float2* Xin, fl
                 const float2 a = cscale(cadd(ck, cm), 0.5f);
                 const float2 d = csub(ck, cm);
                 const float2 b = make_float2(0.5f * d.y, -0.5f * d.x);
-                const float2 k0 = K0[k], kn = KN[k];
+                const float2 k0 = EARLY_K ? kr[EARLY_K ? i : 0] : Kr[k], kn = KN[k];
                 const float2 ak = cmul(a, make_float2(k0.x, ksign * k0.y));
                 const float2 bk = cmul(b, make_float2(kn.x, ksign * kn.y));
                 v[i] = make_float2(ak.x - bk.y, ak.y + bk.x);
             }
         } else {
-            col_kmul<PL>(v, K + (unsigned)(kx * H), t, ksign);
+            col_kmul<PL, EARLY_K>(v, kr, Kr, t, ksign);
         }
         seq_sync<PL>();
     } else {
-        col_kmul<PL>(v, K + (unsigned)(kx * H), t, ksign);
+        col_kmul<PL, EARLY_K>(v, kr, Kr, t, ksign);
     }
 
     fft_regs<PL, +1>(v, row, t, g.twP[PL::variant]);

@@ -121,6 +121,17 @@ def test_every_fft_plan_variant_matches_oracle(fm, orc, case):
         check_rl(out, est, out_o, est_o)
 
 
+@pytest.mark.parametrize("case", [(1, 2, 98, 98, 31, 31),     # 128 x 128 (rows of 64)
+                                  (1, 2, 100, 226, 29, 31),   # 128 x 256, all of the row extent
+                                  (9, 1, 226, 255, 31, 2),    # 256 x 256, more planes than one group
+                                  (3, 2, 227, 470, 21, 21)],  # 256 x 512
+                         ids=lambda c: f"{c[0]}x{c[2]}x{c[3]}")
+def test_small_fft_plan_variants_match_oracle(fm, orc, case):
+    """Rows and columns of 128 and 256 points, where a workgroup holds several: the
+    same tolerance as the longer ones."""
+    test_every_fft_plan_variant_matches_oracle(fm, orc, case)
+
+
 @pytest.mark.parametrize("dh, dw, k", [(64, 80, 15), (1024, 1024, 41)])
 def test_conjugate_kernel_hat_matches_explicit(fm, orc, monkeypatch, dh, dw, k):
     """Independent PSFs of odd size: pass C multiplies by the conjugate of the
