@@ -179,6 +179,7 @@ template <typename S> struct Batch {
                 c.fftH = fftH;
                 c.fftW = fftW;
                 c.N = fftW / 2;
+                c.var = default_variants(c.fftH);
                 cls.push_back(std::move(c));
             }
             v.cls = classOf[key];

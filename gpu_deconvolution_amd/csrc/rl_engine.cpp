@@ -160,6 +160,7 @@ template <typename S> struct Plan {
         fftH = snap_transform_size(dataH + kernelH - 1);
         fftW = snap_transform_size(dataW + kernelW - 1);
         N = fftW / 2;
+        var = default_variants(fftH);
         if (!row_size_supported(N) || !col_size_supported(fftH) || fftW < 16 || fftH < 16) {
             char msg[160];
             snprintf(msg, sizeof msg, "unsupported FFT extent %d x %d (data %d x %d, kernel %d x %d)",
