@@ -455,7 +455,9 @@ template <typename PL> constexpr int tw_pass_offset(int i)
 }
 template <typename PL> constexpr int tw_table_len() { return tw_pass_offset<PL>(PL::NP); }
 
-// Host: the per-pass twiddle table of plan PL.
+template <typename PL> std::vector<float2> base_powers(const std::vector<float2>& table);
+
+// Host: the per-pass twiddle table of plan PL, followed by its base powers (TwLds).
 template <typename PL> std::vector<float2> pass_twiddle_table()
 {
     std::vector<float2> t((size_t)tw_table_len<PL>());
@@ -470,6 +472,8 @@ template <typename PL> std::vector<float2> pass_twiddle_table()
                 t[(size_t)off + (size_t)(r - 1) * NS + k] = make_float2((float)std::cos(a), (float)std::sin(a));
             }
     }
+    const std::vector<float2> b = base_powers<PL>(t);
+    t.insert(t.end(), b.begin(), b.end());
     return t;
 }
 
@@ -823,17 +827,72 @@ __device__ __forceinline__ void inv_passes(float2* v, typename PL::E* lds, int t
     }
 }
 
+// Or from LDS: the base powers w^k and, for radices above 8, w^(Q k), k < NS, of
+// every pass, which the row tiles copy there before the first pass.  A
+// wavefront's global loads return in order, so a pass that reads its twiddles from
+// global memory waits for every load issued before them: in the ratio pass, for the
+// samples that are streamed from HBM behind the tile, at the first pass
+// instead of at their use.  Twiddles held in registers avoid that too, but their 4 to 12
+// registers spilled or cost a resident wavefront in most row plans.
+template <typename PL, int I = 1> constexpr bool tw_all_generated()
+{
+    if constexpr (I >= PL::NP) return true;
+    else if constexpr (!tw_generated<PL, I>()) return false;
+    else return tw_all_generated<PL, I + 1>();
+}
+template <typename PL, int I> constexpr int tw_powers()  // powers of pass I
+{
+    return tw_gen_q<PL::R::at(I)>() < PL::R::at(I) ? 2 * span_before<PL>(I) : span_before<PL>(I);
+}
+template <typename PL, int I> constexpr int tw_power_offset()
+{
+    if constexpr (I <= 1) return 0;
+    else return tw_power_offset<PL, I - 1>() + tw_powers<PL, I - 1>();
+}
+// Number of base powers; 0 where a pass reads the table instead.
+template <typename PL> constexpr int tw_lds_len()
+{
+    if constexpr (tw_all_generated<PL>()) return tw_power_offset<PL, PL::NP>();
+    else return 0;
+}
+template <typename PL> std::vector<float2> base_powers(const std::vector<float2>& table)
+{
+    std::vector<float2> b;
+    if constexpr (tw_lds_len<PL>() > 0)
+        static_for<1, PL::NP>([&]<int I>() {
+            constexpr int NS = span_before<PL>(I), n = tw_powers<PL, I>(), Q = tw_gen_q<PL::R::at(I)>();
+            for (int i = 0; i < n; ++i) b.push_back(table[tw_pass_offset<PL>(I) + (i < NS ? 0 : (Q - 1) * NS) + i % NS]);
+        });
+    return b;
+}
+struct TwLds {
+    const float2* powers;
+};
+template <typename PL, int I> __device__ __forceinline__ void tw_get(float2* w, int t, const TwLds& src)
+{
+    constexpr int R = PL::R::at(I), NS = span_before<PL>(I);
+    if constexpr (NS > 1) {
+        constexpr int Q = tw_gen_q<R>(), NK = tw_shared_k<PL, I>() ? 1 : PL::P / R;
+        const float2* tb = src.powers + tw_power_offset<PL, I>() + tw_k<PL, I>(t, 0);
+        static_for<0, NK>([&]<int b>() {
+            constexpr int d = tw_k<PL, I>(0, b);
+            w[2 * b] = tb[d];
+            if constexpr (Q < R) w[2 * b + 1] = tb[d + NS];
+        });
+    }
+}
+
 // Full unnormalised transform of the sequence owned by T threads, kernel
 // exp(DIR 2 pi i n k / N).  On entry v holds the inputs at the layout
 // "j + r*N/R" of R = first_radix<PL, DIR>() (slot_pos); on exit the outputs,
 // in natural order, at the layout of last_radix<PL, DIR>().  The caller must
 // have ordered any earlier LDS reads of this sequence's slice before the
-// call (seq_sync or a workgroup barrier).  tw: the plan's twiddle table.
-template <typename PL, int DIR>
-__device__ __forceinline__ void fft_regs(float2* v, typename PL::E* lds, int t, const float2* __restrict__ tw)
+// call (seq_sync or a workgroup barrier).  ts: the plan's twiddles (TwTable or TwLds).
+template <typename PL, int DIR, typename TS>
+__device__ __forceinline__ void fft_regs(float2* v, typename PL::E* lds, int t, const TS& ts)
 {
-    if constexpr (DIR < 0) fwd_passes<PL, 0>(v, lds, t, TwTable{tw});
-    else inv_passes<PL, PL::NP - 1>(v, lds, t, TwTable{tw});
+    if constexpr (DIR < 0) fwd_passes<PL, 0>(v, lds, t, ts);
+    else inv_passes<PL, PL::NP - 1>(v, lds, t, ts);
 }
 
 // Position of input r of butterfly b for thread t in the layout of radix R.

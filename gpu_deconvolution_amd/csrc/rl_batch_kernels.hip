@@ -48,13 +48,14 @@ __global__ __launch_bounds__(RowCfg<PL>::THREADS, PL::WPE) void batch_ratio_kern
 {
     using C = RowCfg<PL>;
     __shared__ typename C::E lds[C::G * C::L];
+    __shared__ float2 twl[C::TWN];
     const int lid = (int)xcd_remap(blockIdx.x, gridDim.x);
     const int e = find_entry(list, n, lid);
     const BatchSeg& S = segs[list[e]];
     const int local = lid - list[n + e], nrg = g.H / C::G;
     const int rg = local % nrg, pl = local / nrg;
     const SAMPLE* d = static_cast<const SAMPLE*>(S.data[view]) + (long)pl * S.dstride;
-    ratio_tile<SAMPLE, PL>(seg_geom(g, S), XT + (long)(S.plane0 + pl) * xstride, d, rg * C::G, lds, S.rscale);
+    ratio_tile<SAMPLE, PL>(seg_geom(g, S), XT + (long)(S.plane0 + pl) * xstride, d, rg * C::G, lds, twl, S.rscale);
 }
 
 template <typename PL>
@@ -67,6 +68,7 @@ __global__ __launch_bounds__(RowCfg<PL>::THREADS, PL::WPE) void batch_update_ker
 {
     using C = RowCfg<PL>;
     __shared__ typename C::E lds[C::G * C::L];
+    __shared__ float2 twl[C::TWN];
     const int lid = (int)xcd_remap(blockIdx.x, gridDim.x);
     const int e = find_entry(list, n, lid);
     const BatchSeg& S = segs[list[e]];
@@ -74,7 +76,7 @@ __global__ __launch_bounds__(RowCfg<PL>::THREADS, PL::WPE) void batch_update_ker
     grouped_tile((unsigned)(lid - list[n + e]), g.H / C::G, S.nplanes, rg, pl);
     const long p = S.plane0 + pl;
     update_tile<PL>(seg_geom(g, S), XE + p * xstride, XT + p * xstride, ES + p * estride, S.w[view], rg * C::G,
-                    lds);
+                    lds, twl);
 }
 
 template <typename PL>

@@ -29,10 +29,11 @@ __global__ __launch_bounds__(RowCfg<PL>::THREADS, PL::WPE) void row_ratio_kernel
 {
     using C = RowCfg<PL>;
     __shared__ typename C::E lds[C::G * C::L];
+    __shared__ float2 twl[C::TWN];
     const int nrg = g.H / C::G;
     const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
     const int rg = lid % nrg, p = lid / nrg;
-    ratio_tile<SAMPLE, PL>(g, X + p * xstride, data + p * dstride, rg * C::G, lds, scale);
+    ratio_tile<SAMPLE, PL>(g, X + p * xstride, data + p * dstride, rg * C::G, lds, twl, scale);
 }
 
 // ------------------------------------------------------------------ pass D
@@ -43,11 +44,12 @@ __global__ __launch_bounds__(RowCfg<PL>::THREADS, PL::WPE) void row_update_kerne
 {
     using C = RowCfg<PL>;
     __shared__ typename C::E lds[C::G * C::L];
+    __shared__ float2 twl[C::TWN];
     const int nrg = g.H / C::G;
     const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
     int rg, p;
     grouped_tile(lid, nrg, nplanes, rg, p);
-    update_tile<PL>(g, XE + p * xstride, XC + p * xstride, ES + p * estride, weights, rg * C::G, lds);
+    update_tile<PL>(g, XE + p * xstride, XC + p * xstride, ES + p * estride, weights, rg * C::G, lds, twl);
 }
 
 // ------------------------------------------------------------------ egress
@@ -79,10 +81,11 @@ __global__ __launch_bounds__(RowCfg<PL>::THREADS, PL::WPE) void row_init_kernel(
 {
     using C = RowCfg<PL>;
     __shared__ typename C::E lds[C::G * C::L];
+    __shared__ float2 twl[C::TWN];
     const int nrg = g.H / C::G;
     const unsigned lid = xcd_remap(blockIdx.x, gridDim.x);
     const int rg = lid % nrg, p = lid / nrg;
-    init_tile<PL>(g, XE + p * xstride, ES + p * estride, e0 + p * e0stride, rg * C::G, lds);
+    init_tile<PL>(g, XE + p * xstride, ES + p * estride, e0 + p * e0stride, rg * C::G, lds, twl);
 }
 
 __global__ void const_init_kernel(float2* __restrict__ XE, float* __restrict__ ES, long xstride, long estride,

@@ -119,6 +119,14 @@ template <typename PL_> struct RowCfg {
     // whether a tile's accesses share one address register (see lds_pad below)
     static constexpr bool AFFINE_T = N % 16 == 0 && (T % 16 == 0 || T == 8);
     static constexpr bool AFFINE_I = AFFINE_T && (N / RFI) % 16 == 0, AFFINE_F = AFFINE_T && (N / RLF) % 16 == 0;
+    // twiddles in LDS (TwLds): the FFT's base powers, then exp(-2 pi i p / W), p < T.
+    // Row lengths where that is the faster (ratio / update, us a launch, table then LDS: 512
+    // 41.6 / 53.7, 38.3 / 52.2; 1024 42.6 / 53.1, 42.7 / 51.6; 1280 254.7 / 389.8,
+    // 251.0 / 379.0); at 768 the further LDS reads of its four short passes cost
+    // more (46.7 / 53.9, 49.9 / 56.2), at the other lengths the two are level or so.
+    static constexpr bool TWLDS = (N == 512 || N == 1024 || N == 1280) && tw_lds_len<PL>() > 0 && AFFINE_I && AFFINE_F;
+    static constexpr int TWP = TWLDS ? tw_lds_len<PL>() : 0;
+    static constexpr int TWN = TWLDS ? TWP + T : 1;
 };
 
 // LDS addressing.  With t below T and c a multiple of T, lds_pad(t + c) = lds_pad(t) + c + c/16
@@ -449,29 +457,73 @@ __device__ __forceinline__ void unpack_pair(PairT w, float& a, float& b)
     }
 }
 
+// A row tile's twiddles: the table of exp(-2 pi i p / W) and the FFT's, in LDS
+// where the plan allows it.  prefetch loads this thread's share, store writes it to
+// LDS before the tile's first barrier.
+template <typename C> struct RowTwiddles {
+    using PL = typename C::PL;
+    static constexpr int PER = (C::TWN + C::THREADS - 1) / C::THREADS;
+    float2 r[PER];
+    float2* lds;
+    const RowGeom& g;
+    __device__ __forceinline__ RowTwiddles(const RowGeom& geom, float2* twl, int tid) : lds(twl), g(geom)
+    {
+        if constexpr (C::TWLDS) {
+            const float2* powers = g.twP[PL::variant] + tw_table_len<PL>();
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                const int e = tid + i * C::THREADS;
+                if (e < C::TWN) r[i] = e < C::TWP ? powers[e] : g.twW[e - C::TWP];
+            }
+        }
+    }
+    __device__ __forceinline__ void store(int tid) const
+    {
+        if constexpr (C::TWLDS) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                const int e = tid + i * C::THREADS;
+                if (e < C::TWN) lds[e] = r[i];
+            }
+        }
+    }
+    __device__ __forceinline__ auto fft() const
+    {
+        if constexpr (C::TWLDS) return TwLds{lds};
+        else return TwTable{g.twP[PL::variant]};
+    }
+    __device__ __forceinline__ const float2* w() const
+    {
+        if constexpr (C::TWLDS) return lds + C::TWP;
+        else return g.twW;
+    }
+};
+
 // Inverse real FFT of this thread's row from the tile that v holds (as
 // fetch_tile loaded it): the tile is staged in LDS, the inverse FFT's input
 // formed from it and transformed; on return v holds (f[2n], f[2n+1]) at the
 // positions slot_pos<PL, RLI>.
 template <typename C>
-__device__ __forceinline__ void row_c2r(float2* v, typename C::E* lds, int tid, int seq, int t, const RowGeom& g)
+__device__ __forceinline__ void row_c2r(float2* v, typename C::E* lds, int tid, int seq, int t,
+                                        const RowTwiddles<C>& tw)
 {
     typename C::E* row = lds + seq * C::L;
+    tw.store(tid);
     if constexpr (C::PL::SPLIT) {
-        stage_c2r_pre_split<C>(v, lds, tid, seq, t, g.twW);
+        stage_c2r_pre_split<C>(v, lds, tid, seq, t, tw.w());
     } else {
         stage_tile<C>(lds, v, tid);
         __syncthreads();
-        c2r_pre<C>(v, row, t, g.twW);
+        c2r_pre<C>(v, row, t, tw.w());
     }
     seq_sync<typename C::PL>();
-    fft_regs<typename C::PL, +1>(v, row, t, g.twP[C::PL::variant]);
+    fft_regs<typename C::PL, +1>(v, row, t, tw.fft());
 }
 
 // ------------------------------------------------------------- row tiles
 // Each works on the G rows [y0, y0+G) of one padded plane; lds holds
-// G*RowCfg::L elements.  g carries the FFT extent (uniform over the launch) and the data
-// extent and pad half-widths of the plane's volume.
+// G*RowCfg::L elements, twl RowCfg::TWN twiddles.  g carries the FFT extent (uniform
+// over the launch) and the data extent and pad half-widths of the plane's volume.
 
 // Pass B: X <- R2C(Q > 1 ? D / Q : Q) * scale, Q = C2R(X).  divide_kernel_{16,8},
 // fmvd_deconvolve_cuda.impl.cu:159-176; the data is read unpadded through the
@@ -479,7 +531,8 @@ __device__ __forceinline__ void row_c2r(float2* v, typename C::E* lds, int tid, 
 // is 1, or 1/W when pass C's kernel spectrum is pass A's (which carries 1/H only).
 template <typename SAMPLE, typename PL>
 __device__ __forceinline__ void ratio_tile(const RowGeom& g, float2* __restrict__ Xp,
-                                           const SAMPLE* __restrict__ dplane, int y0, typename PL::E* lds, float scale)
+                                           const SAMPLE* __restrict__ dplane, int y0, typename PL::E* lds,
+                                           float2* twl, float scale)
 {
     using C = RowCfg<PL>;
     using PairT = typename PairOf<SAMPLE>::type;
@@ -488,6 +541,7 @@ __device__ __forceinline__ void ratio_tile(const RowGeom& g, float2* __restrict_
     typename C::E* row = lds + seq * C::L;
     float2 v[C::P];
     fetch_tile<C>(v, Xp, g.H, y0, tid);
+    const RowTwiddles<C> tw(g, twl, tid);
     // the row's samples (streamed from HBM once per view-iteration) are loaded
     // behind the tile, ahead of the FFT, so their latency hides behind it
     const SAMPLE* drow = dplane + (unsigned)(pad_index(y, g.dataH, g.dkY) * g.dataW);
@@ -501,7 +555,7 @@ __device__ __forceinline__ void ratio_tile(const RowGeom& g, float2* __restrict_
         }
     };
     load_samples();
-    row_c2r<C>(v, lds, tid, seq, t, g);
+    row_c2r<C>(v, lds, tid, seq, t, tw);
 #pragma unroll
     for (int i = 0; i < C::P; ++i) {
         const float q0 = v[i].x, q1 = v[i].y;
@@ -511,8 +565,8 @@ __device__ __forceinline__ void ratio_tile(const RowGeom& g, float2* __restrict_
         v[i].x = q0 > 1.0f ? d0 * __builtin_amdgcn_rcpf(q0) : q0;
         v[i].y = q1 > 1.0f ? d1 * __builtin_amdgcn_rcpf(q1) : q1;
     }
-    fft_regs<PL, -1>(v, row, t, g.twP[C::PL::variant]);
-    r2c_post_store<C>(v, lds, Xp, g.H, y0, tid, seq, t, g.twW, scale);
+    fft_regs<PL, -1>(v, row, t, tw.fft());
+    r2c_post_store<C>(v, lds, Xp, g.H, y0, tid, seq, t, tw.w(), scale);
 }
 
 // Pass D: C = C2R(XC); E <- E + w (E C - E) on the spatial estimate (one
@@ -522,7 +576,8 @@ __device__ __forceinline__ void ratio_tile(const RowGeom& g, float2* __restrict_
 template <typename PL>
 __device__ __forceinline__ void update_tile(const RowGeom& g, float2* XEp,
                                             const float2* XCp, float* __restrict__ ESp,
-                                            const float* __restrict__ weights, int y0, typename PL::E* lds)
+                                            const float* __restrict__ weights, int y0, typename PL::E* lds,
+                                            float2* twl)
 {
     using C = RowCfg<PL>;
     const int tid = threadIdx.x, seq = tid / C::T, t = tid % C::T;
@@ -530,7 +585,8 @@ __device__ __forceinline__ void update_tile(const RowGeom& g, float2* XEp,
     typename C::E* row = lds + seq * C::L;
     float2 v[C::P];
     fetch_tile<C>(v, XCp, g.H, y0, tid);
-    row_c2r<C>(v, lds, tid, seq, t, g);
+    const RowTwiddles<C> tw(g, twl, tid);
+    row_c2r<C>(v, lds, tid, seq, t, tw);
 
     float2* erow = reinterpret_cast<float2*>(ESp) + (unsigned)(y * (g.W / 2));
     const float* wrow = weights + (unsigned)(pad_index(y, g.dataH, g.wkY) * g.dataW);
@@ -550,14 +606,14 @@ __device__ __forceinline__ void update_tile(const RowGeom& g, float2* XEp,
         v[i].y = e.y + c1;
         erow[t + c] = v[i];
     }
-    fft_regs<PL, -1>(v, row, t, g.twP[C::PL::variant]);
-    r2c_post_store<C>(v, lds, XEp, g.H, y0, tid, seq, t, g.twW, 1.0f / (float)g.W);
+    fft_regs<PL, -1>(v, row, t, tw.fft());
+    r2c_post_store<C>(v, lds, XEp, g.H, y0, tid, seq, t, tw.w(), 1.0f / (float)g.W);
 }
 
 // Warm-start ingest: ES <- pad(E0) (data pad map), XE <- R2C(ES) / W.
 template <typename PL>
 __device__ __forceinline__ void init_tile(const RowGeom& g, float2* __restrict__ XEp, float* __restrict__ ESp,
-                                          const float* __restrict__ e0p, int y0, typename PL::E* lds)
+                                          const float* __restrict__ e0p, int y0, typename PL::E* lds, float2* twl)
 {
     using C = RowCfg<PL>;
     const int tid = threadIdx.x, seq = tid / C::T, t = tid % C::T;
@@ -565,6 +621,9 @@ __device__ __forceinline__ void init_tile(const RowGeom& g, float2* __restrict__
     typename C::E* row = lds + seq * C::L;
     const float* erow = e0p + (unsigned)(pad_index(y, g.dataH, g.dkY) * g.dataW);
     float2* esrow = reinterpret_cast<float2*>(ESp) + (unsigned)(y * (g.W / 2));
+    const RowTwiddles<C> tw(g, twl, tid);
+    tw.store(tid);
+    if constexpr (C::TWLDS) __syncthreads();
     float2 v[C::P];
 #pragma unroll
     for (int i = 0; i < C::P; ++i) {
@@ -573,8 +632,8 @@ __device__ __forceinline__ void init_tile(const RowGeom& g, float2* __restrict__
         v[i].y = erow[pad_index(2 * n + 1, g.dataW, g.dkX)];
         esrow[n] = v[i];
     }
-    fft_regs<PL, -1>(v, row, t, g.twP[C::PL::variant]);
-    r2c_post_store<C>(v, lds, XEp, g.H, y0, tid, seq, t, g.twW, 1.0f / (float)g.W);
+    fft_regs<PL, -1>(v, row, t, tw.fft());
+    r2c_post_store<C>(v, lds, XEp, g.H, y0, tid, seq, t, tw.w(), 1.0f / (float)g.W);
 }
 
 // ---------------------------------------------------------- column tile
@@ -669,7 +728,7 @@ __device__ __forceinline__ void col_tile(const ColGeom& g, const float2* Xin, fl
     const float2* Kr = K + (unsigned)(kx * H);
     float2 kr[EARLY_K ? C::P : 1];
     if constexpr (EARLY_K) col_kload<PL>(kr, Kr, t);
-    fft_regs<PL, -1>(v, row, t, g.twP[PL::variant]);
+    fft_regs<PL, -1>(v, row, t, TwTable{g.twP[PL::variant]});
 
     if (grp == 0) {  // workgroup-uniform: this group holds the packed DC/Nyquist sequence
         if (seq == 0) {
@@ -700,7 +759,7 @@ __device__ __forceinline__ void col_tile(const ColGeom& g, const float2* Xin, fl
         col_kmul<PL, EARLY_K>(v, kr, Kr, t, ksign);
     }
 
-    fft_regs<PL, +1>(v, row, t, g.twP[PL::variant]);
+    fft_regs<PL, +1>(v, row, t, TwTable{g.twP[PL::variant]});
     float2* xo = Xout + (unsigned)xpos(kx, 0, H);
     const int ts = fresh(t);
 #pragma unroll

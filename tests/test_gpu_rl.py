@@ -261,6 +261,27 @@ def test_warm_start_matches_oracle(fm, orc):
     assert np.abs(e0 - init).max() <= 1e-4 * np.abs(init).max()
 
 
+@pytest.mark.parametrize("dw, k", [(760, 15), (996, 29), (1540, 13), (2018, 31), (2060, 15), (2548, 13)])
+def test_rows_with_twiddles_in_lds(fm, orc, dw, k):
+    """Row lengths whose twiddles are read from LDS, with data that just misses the next
+    shorter extent or fills its own, cold and from a warm start, to the tolerance of the
+    other extents."""
+    Z, V, dh = 1, 2, 20
+    data, kernels, weights = make_case(Z, V, dh, dw, 13, k, 16, seed=dw)
+    out, est, _ = run_gpu(fm, data, kernels, weights, 0, 2, 16)
+    out_o, est_o = orc.rl_planes(data, weights, kernels.copy(), 0, 2, threads=8)
+    check_rl(out, est, out_o, est_o)
+    init = np.random.default_rng(dw).uniform(50, 400, size=(Z, dh, dw)).astype(np.float32)
+    out_o, est_o = orc.rl_planes(data, weights, kernels.copy(), 0, 2, init=init.astype(np.float64))
+    views, dinit, dest = [to_device(np.ascontiguousarray(data[:, v])) for v in range(V)], to_device(init), \
+        empty_device((Z, dh, dw), np.float32)
+    dout = empty_device((Z, dh, dw), np.uint16)
+    with fm.Deconvolver(dh, dw, list(weights), [x.copy() for x in kernels]) as dec:
+        dec.run_device([t.ptr for t in views], Z, 2, out_ptr=dout.ptr, est_ptr=dest.ptr, init_ptr=dinit.ptr, stream=0)
+        fm.device_synchronize()
+    check_rl(from_device(dout, np.uint16), from_device(dest, np.float32), out_o, est_o)
+
+
 def test_invalid_device_reports_error(fm):
     fm.lib().setCudaDevice(97)
     errs = fm.take_errors()
