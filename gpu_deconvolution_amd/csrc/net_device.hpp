@@ -47,5 +47,18 @@ __device__ __forceinline__ unsigned xcd_block(unsigned bid, unsigned nblocks)
 // the column alone, so rows are immediate offsets.
 __device__ __forceinline__ int slot_swizzle(int c) { return (c & 2) | ((c >> 2) & 1); }
 
+// A voxel's 32 channels, held as bf16 pairs c[q][i] = channels 8 q + 4 (lane / 32) + 2 i, + 1 by
+// the lanes l and l + 32: each lane gets two 16-byte pieces (channels 8 q .. 8 q + 7 for q =
+// lane / 32 and 2 + lane / 32) and stores them.
+__device__ __forceinline__ void store_voxel(uint16_t* __restrict__ v, const uint32_t (*c)[2], int kh)
+{
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const auto a = __builtin_amdgcn_permlane32_swap(c[2 * h][0], c[2 * h + 1][0], false, false);
+        const auto b = __builtin_amdgcn_permlane32_swap(c[2 * h][1], c[2 * h + 1][1], false, false);
+        reinterpret_cast<uint4*>(v)[2 * h + kh] = make_uint4(a[0], b[0], a[1], b[1]);
+    }
+}
+
 }  // namespace net
 }  // namespace fmvd

@@ -9,8 +9,8 @@
 //
 // The four 32->32 layers (98% of the work) run on MFMA (net_conv32.hip), their
 // weight gradients and those of the edge layers too (net_wgrad.hip).  The
-// 2->32 input layer and the 32->1 output layer have too few channels for MFMA
-// tiles and run on the VALU, still with FP32 accumulation.
+// 2->32 input layer and the 32->1 output layer's input gradient use the FP32
+// matrix instruction; the output layer has one channel and runs on the VALU.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -72,46 +72,108 @@ __global__ void prep_input_kernel(const uint16_t* const* __restrict__ views, int
     x[2 * (n * per + i) + 1] = f2bf(o * k);
 }
 
-// The edge layers run on the VALU.
+// The input layer and the output layer's input gradient take one dword of each neighbour
+// and give 32 channels: a block stages the box of kEZ x kEY x kEX voxels with its halo
+// in LDS once, and a wavefront computes rows of 32 voxels on MFMA.  Walking planes
+// would save only re-reads of the halo (0.8 dwords a voxel next to the 16 and 48 written).
+constexpr int kEX = 32, kEY = 16, kEZ = 4, kEThreads = 256;
+constexpr int kEHX = kEX + 2, kEHY = kEY + 2, kEHZ = kEZ + 2, kEBox = kEHZ * kEHY * kEHX;
 
-// Layer 1 (2 -> 32): h1 = relu(conv(x, W1) + b1); W1 is FP32 [27][32][2]
-// (bf16-rounded values).  One thread per voxel; relu (if wanted): the bits h1 > 0.
-// Bound by the VALU: 27 x 32 x 3 instructions a voxel (two products, rounded
-// separately, and their sum) are 553 us at 8 x 64 x 128 x 128, measured 634; reading the
-// weights through scalar loads, or walking planes with 96 sums a thread to
-// read a neighbour once, measured 656 and 734.
-__global__ void conv_in_kernel(const uint16_t* __restrict__ x, Geo g, const float* __restrict__ w,
-                               const float* __restrict__ b, uint16_t* __restrict__ h,
-                               uint32_t* __restrict__ relu)
+struct EdgeTile {
+    int n, z, y, x;
+};
+__device__ __forceinline__ EdgeTile edge_tile(const Geo& g)
 {
-    __shared__ float ws[27 * 32 * 2 + 32];
-    for (int i = threadIdx.x; i < 27 * 64 + 32; i += blockDim.x) ws[i] = i < 27 * 64 ? w[i] : b[i - 27 * 64];
+    const int nx = (g.W + kEX - 1) / kEX, ny = (g.H + kEY - 1) / kEY, nz = (g.D + kEZ - 1) / kEZ;
+    int b = (int)xcd_block(blockIdx.x, gridDim.x);
+    EdgeTile t;
+    t.x = b % nx * kEX;
+    b /= nx;
+    t.y = b % ny * kEY;
+    b /= ny;
+    t.z = b % nz * kEZ;
+    t.n = b / nz;
+    return t;
+}
+template <typename Put>
+__device__ __forceinline__ void load_box(const uint32_t* __restrict__ in, const Geo& g, const EdgeTile& t, Put put)
+{
+    constexpr int kLoads = (kEBox + kEThreads - 1) / kEThreads;
+    uint32_t r[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int e = threadIdx.x + kEThreads * i;
+        const int z = t.z + e / (kEHY * kEHX) - 1, y = t.y + e / kEHX % kEHY - 1, x = t.x + e % kEHX - 1;
+        r[i] = 0;
+        if (e < kEBox && z >= 0 && z < g.D && y >= 0 && y < g.H && x >= 0 && x < g.W) r[i] = in[g.vox(t.n, z, y, x)];
+    }
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int e = threadIdx.x + kEThreads * i;
+        if (e < kEBox) put(e, r[i]);
+    }
+}
+// position in the box, relative to its first voxel, of the neighbour that a tap reads
+__device__ constexpr int box_offset(int tap) { return (tap / 9 * kEHY + tap / 3 % 3) * kEHX + tap % 3; }
+
+// Layer 1 (2 -> 32): h1 = relu(conv(x, W1) + b1); W1 is FP32 [27][32][2] (bf16-rounded
+// values).  relu (if wanted): the bits h1 > 0.  A tap's two products and their FP32 sum are one
+// v_mfma_f32_32x32x2_f32 from zero, which the VALU adds to the taps' sum in their order: the
+// rounding of the definition.  (The bf16 instruction would take all 54 products in 4 steps, but it
+// truncates inside a sum: 5 % of two-product sums differ in their last bit.)
+// Weights and inputs are finite (taps outside the volume multiply by zero).
+// At 8 x 64 x 128 x 128: 619 us on the VALU (three instructions a tap and channel, 553 us of issue),
+// 470 here: a tap's 64 cycles of products and 64 of additions a wavefront do not overlap
+// (368 us; issuing the next tap's products first changed nothing).  At most 128 registers,
+// or the products land in accumulation registers and a copy each costs a third again (585 us).
+__global__ __launch_bounds__(kEThreads, 4) void conv_in_kernel(const uint32_t* __restrict__ x, Geo g,
+                                                               const float* __restrict__ w,
+                                                               const float* __restrict__ b,
+                                                               uint16_t* __restrict__ h, uint32_t* __restrict__ relu)
+{
+    __shared__ uint32_t box[2 * kEBox];  // FP32: channel 0, channel 1
+    const EdgeTile t = edge_tile(g);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 31, kh = lane >> 5;
+    float wk[27];
+#pragma unroll
+    for (int k = 0; k < 27; ++k) wk[k] = w[(k * 32 + m) * 2 + kh];
+    f32x16 bias;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bias[r] = b[8 * (r / 4) + 4 * kh + r % 4];
+    load_box(x, g, t, [&](int e, uint32_t v) {
+        box[e] = v << 16;
+        box[kEBox + e] = v & 0xffff0000u;
+    });
     __syncthreads();
-    const long per = (long)g.D * g.H * g.W;
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int n = blockIdx.y;
-    if (i >= per) return;
-    const int xx = (int)(i % g.W), yy = (int)((i / g.W) % g.H), zz = (int)(i / ((long)g.W * g.H));
-    float acc[32];
+    const int xx = t.x + m;
+    for (int row = wave; row < kEZ * kEY; row += kEThreads / 64) {
+        const int dz = row / kEY, dy = row % kEY, zz = t.z + dz, yy = t.y + dy;
+        if (zz >= g.D || yy >= g.H) continue;  // wave-uniform
+        const uint32_t* v0 = box + kh * kEBox + (dz * kEHY + dy) * kEHX + m;
+        f32x16 acc = bias;
 #pragma unroll
-    for (int c = 0; c < 32; ++c) acc[c] = ws[27 * 64 + c];
-    for (int k = 0; k < 27; ++k) {
-        const int z = zz + k / 9 - 1, y = yy + (k / 3) % 3 - 1, xi = xx + k % 3 - 1;
-        if (z < 0 || z >= g.D || y < 0 || y >= g.H || xi < 0 || xi >= g.W) continue;
-        const long v = g.vox(n, z, y, xi);
-        const float x0 = bf2f(x[2 * v]), x1 = bf2f(x[2 * v + 1]);
+        for (int k = 0; k < 27; ++k)
+            acc += __builtin_amdgcn_mfma_f32_32x32x2f32(wk[k], __uint_as_float(v0[box_offset(k)]), f32x16{}, 0, 0, 0);
+        uint32_t c[4][2], pos = 0;
 #pragma unroll
-        for (int c = 0; c < 32; ++c) acc[c] += x0 * ws[(k * 32 + c) * 2] + x1 * ws[(k * 32 + c) * 2 + 1];
+        for (int q = 0; q < 4; ++q) {
+            uint16_t o[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                o[i] = f2bf(fmaxf(acc[4 * q + i], 0.f));
+                if (o[i]) pos |= 1u << (8 * q + 4 * kh + i);
+            }
+            c[q][0] = o[0] | (uint32_t)o[1] << 16;
+            c[q][1] = o[2] | (uint32_t)o[3] << 16;
+        }
+        const auto both = __builtin_amdgcn_permlane32_swap(pos, pos, false, false);
+        // (lanes l and l + 32 hold one voxel: they leave together)
+        if (xx < g.W) {
+            const long v = g.vox(t.n, zz, yy, xx);
+            store_voxel(h + v * kC, c, kh);
+            if (relu && kh == 0) relu[v] = both[0] | both[1];
+        }
     }
-    uint16_t* o = h + (n * per + i) * 32;
-    uint32_t pos = 0;
-#pragma unroll
-    for (int c = 0; c < 32; ++c) {
-        const uint16_t r = f2bf(fmaxf(acc[c], 0.f));
-        if (r) pos |= 1u << c;
-        o[c] = r;
-    }
-    if (relu) relu[n * per + i] = pos;
 }
 
 // Layer 6 (32 -> 1): y = conv(h5, W6) + b6 + (x0 + x1) / 2 (FP32 out).  A block
@@ -220,37 +282,65 @@ __global__ void loss_kernel(const float* __restrict__ y, const float* __restrict
     if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// dh5[v][c] = sum_k dy[v - off(k)] W6[k][c]  (FP32 out), and the masked bf16
-// gradient of layer 5 (relu: its bits r > 0)
-__global__ void out_dgrad_kernel(const float* __restrict__ dy, Geo g, const float* __restrict__ w,
-                                 const uint32_t* __restrict__ relu, float* __restrict__ dh,
-                                 uint16_t* __restrict__ gout)
+// dh5[v][c] = sum_k dy[v - off(k)] W6[k][c]  (FP32 out), and the masked bf16 gradient of
+// layer 5 (relu: its bits r > 0).  Products and sums are FP32: v_mfma_f32_32x32x2_f32, two
+// taps at a time in the order dz, dy, dx.  The masks are staged too: a load between the rows
+// would wait for the stores of the row before it.
+// At 8 x 64 x 128 x 128 (1.68 GB moved): 719 us with a voxel per thread, whose 128 and 64 bytes
+// left in pieces, 490 here (3.4 TB/s); 554 with the masks loaded row by row.
+__global__ __launch_bounds__(kEThreads, 4) void out_dgrad_kernel(const uint32_t* __restrict__ dy, Geo g,
+                                                                 const float* __restrict__ w,
+                                                                 const uint32_t* __restrict__ relu,
+                                                                 float* __restrict__ dh, uint16_t* __restrict__ gout)
 {
-    __shared__ float ws[27 * 32];
-    for (int i = threadIdx.x; i < 27 * 32; i += blockDim.x) ws[i] = w[i];
-    __syncthreads();
-    const long per = (long)g.D * g.H * g.W;
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int n = blockIdx.y;
-    if (i >= per) return;
-    const int xx = (int)(i % g.W), yy = (int)((i / g.W) % g.H), zz = (int)(i / ((long)g.W * g.H));
-    float acc[32];
+    __shared__ uint32_t box[kEBox], mask[kEZ * kEY * kEX];
+    const EdgeTile t = edge_tile(g);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 31, kh = lane >> 5;
+    float wk[14];
+    int off[14];
 #pragma unroll
-    for (int c = 0; c < 32; ++c) acc[c] = 0.f;
-    for (int k = 0; k < 27; ++k) {
-        const int z = zz - (k / 9 - 1), y = yy - ((k / 3) % 3 - 1), xi = xx - (k % 3 - 1);
-        if (z < 0 || z >= g.D || y < 0 || y >= g.H || xi < 0 || xi >= g.W) continue;
-        const float d = dy[g.vox(n, z, y, xi)];
-#pragma unroll
-        for (int c = 0; c < 32; ++c) acc[c] += d * ws[k * 32 + c];
+    for (int i = 0; i < 14; ++i) {
+        const int tap = 2 * i + kh;
+        wk[i] = tap < 27 ? w[tap * 32 + m] : 0.f;
+        off[i] = kh ? box_offset(2 * i + 1 < 27 ? 25 - 2 * i : 0) : box_offset(26 - 2 * i);
     }
-    float* o = dh + (n * per + i) * 32;
-    uint16_t* go = gout + (n * per + i) * 32;
-    const uint32_t bits = relu[n * per + i];
+    uint32_t mk[kEZ * kEY * kEX / kEThreads];
 #pragma unroll
-    for (int c = 0; c < 32; ++c) {
-        o[c] = acc[c];
-        go[c] = (bits >> c) & 1 ? f2bf(acc[c]) : (uint16_t)0;
+    for (int i = 0; i < kEZ * kEY * kEX / kEThreads; ++i) {
+        const int e = threadIdx.x + kEThreads * i, z = t.z + e / (kEY * kEX), y = t.y + e / kEX % kEY, x = t.x + e % kEX;
+        mk[i] = z < g.D && y < g.H && x < g.W ? relu[g.vox(t.n, z, y, x)] : 0;
+    }
+    load_box(dy, g, t, [&](int e, uint32_t v) { box[e] = v; });
+#pragma unroll
+    for (int i = 0; i < kEZ * kEY * kEX / kEThreads; ++i) mask[threadIdx.x + kEThreads * i] = mk[i];
+    __syncthreads();
+    const int xx = t.x + m;
+    for (int row = wave; row < kEZ * kEY; row += kEThreads / 64) {
+        const int dz = row / kEY, ry = row % kEY, zz = t.z + dz, yy = t.y + ry;
+        if (zz >= g.D || yy >= g.H) continue;  // wave-uniform
+        const long v = g.vox(t.n, zz, yy, xx);
+        const uint32_t bits = mask[row * kEX + m];
+        const uint32_t* v0 = box + (dz * kEHY + ry) * kEHX + m;
+        f32x16 acc = {};
+#pragma unroll
+        for (int i = 0; i < 14; ++i) {
+            float d = __uint_as_float(v0[off[i]]);
+            if (i == 13 && kh) d = 0.f;
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wk[i], d, acc, 0, 0, 0);
+        }
+        uint32_t c[4][2];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            uint16_t o[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = (bits >> (8 * q + 4 * kh + i)) & 1 ? f2bf(acc[4 * q + i]) : (uint16_t)0;
+            c[q][0] = o[0] | (uint32_t)o[1] << 16;
+            c[q][1] = o[2] | (uint32_t)o[3] << 16;
+            if (xx < g.W)
+                reinterpret_cast<float4*>(dh + v * kC)[2 * q + kh] =
+                    make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+        }
+        if (xx < g.W) store_voxel(gout + v * kC, c, kh);
     }
 }
 
@@ -356,11 +446,17 @@ void launch_pack_weights(const float* params, uint16_t* wf, uint16_t* wt, float*
     pack_weights_kernel<<<nblk(4 * kConv32, 256), 256, 0, s>>>(params, wf, wt, small);
     FMVD_LAUNCH_CHECK();
 }
+static unsigned edge_blocks(Dims d)
+{
+    const long n = (long)d.N * ((d.D + kEZ - 1) / kEZ) * ((d.H + kEY - 1) / kEY) * ((d.W + kEX - 1) / kEX);
+    if (n > 0x7fffffffL) throw_msg("network: volume too large");
+    return (unsigned)n;
+}
 void launch_conv_in(const uint16_t* x, Dims d, const float* small, const float* params, uint16_t* h,
                     uint32_t* relu, hipStream_t s)
 {
-    const long per = (long)d.D * d.H * d.W;
-    conv_in_kernel<<<dim3(nblk(per, 256), d.N), 256, 0, s>>>(x, geo(d), small, params + off_b(0), h, relu);
+    conv_in_kernel<<<edge_blocks(d), kEThreads, 0, s>>>(reinterpret_cast<const uint32_t*>(x), geo(d), small,
+                                                        params + off_b(0), h, relu);
     FMVD_LAUNCH_CHECK();
 }
 void launch_conv_out(const uint16_t* h, const uint16_t* x, Dims d, const float* small, const float* params, float* y,
@@ -384,8 +480,8 @@ int launch_loss(const float* y, const float* t, long count, float* dy, double* p
 void launch_out_dgrad(const float* dy, Dims d, const float* small, const uint32_t* relu, float* dh, uint16_t* gout,
                       hipStream_t s)
 {
-    const long per = (long)d.D * d.H * d.W;
-    out_dgrad_kernel<<<dim3(nblk(per, 256), d.N), 256, 0, s>>>(dy, geo(d), small + 27 * 64, relu, dh, gout);
+    out_dgrad_kernel<<<edge_blocks(d), kEThreads, 0, s>>>(reinterpret_cast<const uint32_t*>(dy), geo(d), small + 27 * 64,
+                                                          relu, dh, gout);
     FMVD_LAUNCH_CHECK();
 }
 void launch_adam(float* p, const float* g, float* m, float* v, int count, float lr, int step, hipStream_t s)

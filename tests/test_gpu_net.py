@@ -155,3 +155,22 @@ def test_gradients_at_tile_edges(fm, shape):
         for i in range(2):
             d, n = np.linalg.norm(gg[l][i] - grads_o[l][i]), np.linalg.norm(grads_o[l][i])
             assert d <= 2e-2 * n + 1e-7, (l, i, d, n)
+
+
+@pytest.mark.parametrize("shape", [(1, 4, 16, 32), (2, 5, 17, 33), (1, 9, 33, 65), (3, 8, 15, 24)])
+def test_edge_layers_at_box_edges(fm, shape):
+    """Input layer and the output layer's input gradient at the edges of their 4 x 16 x 32 boxes.  With the blocks'
+    weights and biases zero the network is h5 = relu(conv(x)), y = conv(h5): the output is one FP32 sum of bfloat16
+    products, so it differs from FP64 by FP32 sums of 27 x 32 terms (1e-6) and rare flips of a bfloat16 rounding
+    (2^-8 each); an h1 or a neighbour taken from elsewhere changes it by its own size."""
+    params, x, t = make_problem(31, shape)
+    for l in range(1, 5):
+        params[l][0][...] = 0.0
+        params[l][1][...] = 0.0
+    net, y, loss, g = run_gpu(fm, params, x, t)
+    loss_o, grads_o, y_o = oracle_batch(params, x, t)
+    assert np.abs(y - y_o).max() <= 2e-3 * np.abs(y_o).max()
+    gg = unflat(g)
+    for l in (0, 5):
+        for i in range(2):
+            assert np.linalg.norm(gg[l][i] - grads_o[l][i]) <= 5e-3 * np.linalg.norm(grads_o[l][i]), (l, i)
