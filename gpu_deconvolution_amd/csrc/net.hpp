@@ -48,7 +48,7 @@ void launch_conv32_fwd(const uint16_t* in, Dims d, const uint16_t* wf_layer, con
 void launch_conv32_dgrad(const uint16_t* g, Dims d, const uint16_t* wt_layer, const uint32_t* relu, float* dh,
                          bool keep_dh, uint16_t* gout, hipStream_t s);
 void launch_conv_out(const uint16_t* h, const uint16_t* x, Dims d, const float* small, const float* params, float* y,
-                     hipStream_t s);
+                     bool training, hipStream_t s);
 // loss partial sums (FP64, one per block of the returned count) and dy
 int launch_loss(const float* y, const float* t, long count, float* dy, double* partial, hipStream_t s);
 void launch_out_dgrad(const float* dy, Dims d, const float* small, const uint32_t* relu, float* dh, uint16_t* gout,

@@ -106,7 +106,7 @@ struct Engine {
                               training ? relu[l].as<uint32_t>() : nullptr, out, s);
         }
         const uint16_t* h5 = training ? h[4].as<uint16_t>() : h[0].as<uint16_t>();
-        launch_conv_out(h5, X, d, small.as<float>(), P, y.as<float>(), s);
+        launch_conv_out(h5, X, d, small.as<float>(), P, y.as<float>(), training, s);
     }
 
     // Gradients of mean((y - t)^2); returns the loss (FP64 sums on the GPU).

@@ -174,3 +174,33 @@ def test_edge_layers_at_box_edges(fm, shape):
     for l in (0, 5):
         for i in range(2):
             assert np.linalg.norm(gg[l][i] - grads_o[l][i]) <= 5e-3 * np.linalg.norm(grads_o[l][i]), (l, i)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (16, 8, 32), (17, 9, 33), (33, 23, 66)])
+def test_inference_output_layer(fm, shape):
+    """Inference's output layer at the edges of its 8 x 32 columns and 16-plane segments, against the oracle and
+    against the training path's chain of FP32 sums of the same activations.  The input is small integers (exact in
+    bfloat16) and the blocks' weights are zero, so both paths see the same h5; sums of 27 x 32 products in FP32
+    differ by at most 864 roundings of 2^-24 of the sum of magnitudes (the oracle with |W6| gives it)."""
+    rng = np.random.default_rng(17)
+    params, _, _ = make_problem(31, (1,) + shape)
+    for l in range(1, 5):
+        params[l][0][...] = 0.0
+        params[l][1][...] = 0.0
+    view = rng.integers(1, 9, size=shape).astype(np.uint16)
+    net = fm.Net(1)
+    net.set_params(flat(params))
+    got = fm.DeviceArray(shape, np.float32)
+    net.infer([fm.DeviceArray.from_host(view)], 1.0, got, floor_value=-1e30)
+    x = np.stack([view, view], -1).astype(np.float64)[None]
+    chain = fm.DeviceArray((1,) + shape, np.float32)
+    net.forward(fm.DeviceArray.from_host(fm.to_bf16_bits(x)), (1,) + shape, chain)
+    fm.device_synchronize()
+    got, chain = got.download(), chain.download()[0]
+    want, _ = onet.forward(params, x[0], quant=True)
+    err, ref = np.abs(got - want), np.abs(chain - want)
+    print(f"{shape}: rms {np.sqrt(np.mean(err**2)):.2e} (chain {np.sqrt(np.mean(ref**2)):.2e}), max {err.max():.2e}")
+    params[5][0] = np.abs(params[5][0])
+    magnitude = np.abs(onet.forward(params, x[0], quant=True)[0]).max()
+    assert np.abs(got.astype(np.float64) - chain).max() <= 864 * 2.0**-24 * magnitude
+    assert err.max() <= 2e-3 * np.abs(want).max()
