@@ -273,7 +273,7 @@ __global__ __launch_bounds__(256) void conv_out_kernel(const uint16_t* __restric
 // P[tap][voxel]: a lane's operands are 16-byte pieces of a voxel, loaded from global
 // memory one plane ahead.  P goes through LDS, and a thread adds the 27 that belong to the
 // outputs p + 1, p, p - 1 of its voxel, in the order dz, dy, dx.  Over 96 x 300 x 260:
-// 463 us with the chains, 200 here; the error of y against 64 bits falls (rms 0.97e-6 against
+// 463 us with the chains, 157 here; the error of y against 64 bits falls (rms 0.97e-6 against
 // 1.31e-6 at 8 x 24 x 40 with |y| to 232 and the same h5, 1.47e-6 against 2.44e-6 with another).
 constexpr int kOThreads = kOY * kOX;
 constexpr int kOGroups = (kOHV + 31) / 32, kOWaves = kOThreads / 64, kOPer = (kOGroups + kOWaves - 1) / kOWaves;
