@@ -11,7 +11,7 @@
 // column (1.33 times with the halo) and used for all 27 taps from LDS; the next
 // step's planes load into registers while the current one multiplies.  The
 // steps are dealt evenly, so the last round of blocks is as full as the
-// first.  The operands stay voxel-major: a matrix operand with the voxels along
+// first.  The operands stay voxel-major: a bf16 matrix operand with the voxels along
 // its reduction dimension is read from them by ds_read_b64_tr_b16, which
 // transposes 4 voxels x 16 channels of a 16-lane group, at any voxel
 // offset, so a tap's shift costs an address and no data movement.
@@ -35,7 +35,6 @@ constexpr int kVB = 2 * kC;                  // bytes of one 32-channel voxel
 constexpr int kTileBytes = kWY * kWX * kVB;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
 
 // Column of steps: sample, first row, first voxel.
 struct Column {
@@ -230,11 +229,15 @@ __device__ __forceinline__ uint32_t load_halo_word(const uint32_t* __restrict__ 
 }
 
 // --------------------------------------------------------------- input layer
-// 32 x (27 taps x 2 channels): B holds the 54 (tap, channel) pairs, a column
-// of ones (the bias) and zeros, in two 32-column tiles.  x lies channel-major in
-// LDS, so that a lane's 8 voxels of one pair are 8 consecutive 16-bit words.
-constexpr int kXPlane = kHY * 2 * kPitch;  // 16-bit words of one plane of x
-constexpr int kXBytes = 3 * kXPlane * 2;
+// 32 x (27 taps x 2 channels) with the FP32 matrix instruction, two voxels at a time: B holds
+// the 54 (tap, channel) pairs, a column of ones (the bias) and zeros, in two 32-column tiles.
+// The bf16 instruction takes 159 us at 8 x 64 x 128 x 128 where this takes 378 (its matrix
+// instructions alone 218), but it cuts low bits off the addends of its sums: gradients with addends
+// of both signs came out up to 2.8 times as far from 64 bits as FP32 sums by rows, these 0.4 to 1.0 times.
+// x lies channel-major in LDS, in FP32.  A step's row of 32 voxels is summed from zero, as
+// in the output layer below.
+constexpr int kXPlane = kHY * 2 * kPitch;  // floats of one plane of x
+constexpr int kXBytes = 3 * kXPlane * 4;
 constexpr int kWgradInLds = 8 * 2 * 16 * 64 * 4;
 static_assert(kXBytes + kTileBytes <= kWgradInLds);
 __global__ __launch_bounds__(kWThreads, 4) void wgrad_in_kernel(const uint16_t* __restrict__ gin,
@@ -243,29 +246,31 @@ __global__ __launch_bounds__(kWThreads, 4) void wgrad_in_kernel(const uint16_t* 
 {
     __shared__ __attribute__((aligned(16))) char lds[kWgradInLds];
     char* const tile = lds + kXBytes;
-    uint16_t* const xs = reinterpret_cast<uint16_t*>(lds);
+    float* const xs = reinterpret_cast<float*>(lds);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned b = xcd_block(blockIdx.x, gridDim.x);
     const int s0 = (int)((long)steps * b / gridDim.x), s1 = (int)((long)steps * (b + 1) / gridDim.x);
+    const int m = lane & 31, kh = lane >> 5;
 
     int base[2], dz[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const int e = t * 32 + (lane & 31), k = e < 54 ? e >> 1 : 0;
+        const int e = t * 32 + m, k = e < 54 ? e >> 1 : 0;
         dz[t] = k / 9;
-        base[t] = ((k / 3 % 3 + wave) * 2 + (e & 1)) * kPitch + k % 3 + 8 * (lane >> 5);
+        base[t] = ((k / 3 % 3 + wave) * 2 + (e & 1)) * kPitch + k % 3 + kh;
     }
-    const bool pair = (lane & 31) < 22;  // of the second tile's columns: pairs 32 .. 53
-    const short fill = (lane & 31) == 22 ? (short)0x3F80 : (short)0;
-    const int offg[2] = {tr_offset(0, 0) + wave * kWX * kVB, tr_offset(0, 1) + wave * kWX * kVB};
+    const bool pair = m < 22;  // of the second tile's columns: pairs 32 .. 53
+    const float fill = m == 22 ? 1.f : 0.f;
+    // g of voxel 2 q + kh: its slot's swizzle depends on q alone (kh is bit 0 of the column)
+    const int gbase = (wave * kWX + kh) * kVB + (m & 7) * 2;
     f32x16 acc[2] = {f32x16{}, f32x16{}};
 
     auto put = [&](int z, uint32_t w) {
         const int v = threadIdx.x;
         if (v >= kHY * kHX) return;
-        uint16_t* d = xs + (z + 3) % 3 * kXPlane + v / kHX * 2 * kPitch + v % kHX;
-        d[0] = (uint16_t)w;
-        d[kPitch] = (uint16_t)(w >> 16);
+        float* d = xs + (z + 3) % 3 * kXPlane + v / kHX * 2 * kPitch + v % kHX;
+        d[0] = __uint_as_float(w << 16);
+        d[kPitch] = __uint_as_float(w & 0xffff0000u);
     };
     uint4 rt[kTilePieces];
     Column c{};
@@ -285,18 +290,22 @@ __global__ __launch_bounds__(kWThreads, 4) void wgrad_in_kernel(const uint16_t* 
             rw = load_halo_word(x, g, c, z + 2);
             load_tile(rt, gin, g, c, z + 1);
         }
+        const float* xr[2];
+        f32x16 row[2] = {f32x16{}, f32x16{}};
 #pragma unroll
-        for (int q = 0; q < kWX; q += 16) {
-            const bf16x8 av = read_tr(tile, offg[0] + q * kVB, offg[1] + q * kVB);
+        for (int t = 0; t < 2; ++t) xr[t] = xs + (z + dz[t] + 2) % 3 * kXPlane + base[t];
+#pragma unroll
+        for (int q = 0; q < kWX / 2; ++q) {
+            const float gv = bf2f(*reinterpret_cast<const uint16_t*>(
+                tile + gbase + 2 * q * kVB + (((m >> 3) ^ slot_swizzle(2 * q)) << 4)));
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
-                const uint16_t* xr = xs + (z + dz[t] + 2) % 3 * kXPlane + base[t] + q;
-                s16x8 v;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) v[j] = (t == 1 && !pair) ? fill : (short)xr[j];
-                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, __builtin_bit_cast(bf16x8, v), acc[t], 0, 0, 0);
+                const float xv = xr[t][2 * q];
+                row[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(gv, t == 1 && !pair ? fill : xv, row[t], 0, 0, 0);
             }
         }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) acc[t] += row[t];
         if (next) {
             __syncthreads();
             put(z + 2, rw);
@@ -325,7 +334,11 @@ __global__ __launch_bounds__(kWThreads, 4) void wgrad_in_kernel(const uint16_t* 
 // -------------------------------------------------------------- output layer
 // dW6[k][ci] = sum_u dy[u - off(k)] h5[u][ci] with dy in FP32: the FP32 matrix
 // instruction v_mfma_f32_32x32x2_f32 (A = 27 shifted dy of 32 rows, B = h5), two
-// voxels at a time, keeps the products and sums in FP32 without splitting dy.
+// voxels at a time, keeps the products and sums in FP32 without splitting dy.  A step's
+// row of 32 voxels is summed from zero and added to the block's sums: with S steps a block, the
+// rounding error of a weight grows like sqrt(32 + S) of a product's, where one chain over
+// all of a block's voxels has sqrt(32 S) (against 64 bits 3 to 5 times as far off; 225 us a launch at
+// 8 x 64 x 128 x 128, 228 with the additions).
 constexpr int kYPlane = kHY * kPitch;
 constexpr int kYBytes = 3 * kYPlane * 4;
 constexpr int kWgradOutLds = 8 * 16 * 64 * 4;
@@ -370,12 +383,14 @@ __global__ __launch_bounds__(kWThreads, 4) void wgrad_out_kernel(const uint32_t*
             load_tile(rt, h5, g, c, z + 1);
         }
         const float* yr = ys + (z + 4 - k / 9) % 3 * kYPlane + ybase;
+        f32x16 row = {};
 #pragma unroll
         for (int q = 0; q < kWX / 2; ++q) {
             const uint16_t h = *reinterpret_cast<const uint16_t*>(
                 tile + hbase + 2 * q * kVB + (((ci >> 3) ^ slot_swizzle(2 * q)) << 4));
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(yr[2 * q], bf2f(h), acc, 0, 0, 0);
+            row = __builtin_amdgcn_mfma_f32_32x32x2f32(yr[2 * q], bf2f(h), row, 0, 0, 0);
         }
+        acc += row;
         if (threadIdx.x < kWY * kWX)
             bsum += ys[z % 3 * kYPlane + ((threadIdx.x >> 5) + 1) * kPitch + (threadIdx.x & 31) + 1];
         if (next) {
@@ -438,12 +453,12 @@ static int wgrad_steps(Dims d)
     return (int)s;
 }
 
-// Blocks (rows of partial sums): one or more per CU, and no fewer than (n, z)
-// planes up to 1024, so that a partial sum covers about one plane of voxels.
+// Blocks (rows of partial sums, added in FP64): one or more per CU, and no fewer than (n, z)
+// planes, so that a partial sum covers at most about one plane of voxels.
 int wgrad_blocks(Dims d)
 {
     const long planes = (long)d.N * d.D;
-    const long nb = (std::min<long>(std::max<long>(planes, 256), 1024) + 255) / 256 * 256;
+    const long nb = (std::max<long>(planes, 256) + 255) / 256 * 256;
     return (int)std::min<long>(nb, wgrad_steps(d));
 }
 

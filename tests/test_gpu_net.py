@@ -204,3 +204,60 @@ def test_inference_output_layer(fm, shape):
     magnitude = np.abs(onet.forward(params, x[0], quant=True)[0]).max()
     assert np.abs(got.astype(np.float64) - chain).max() <= 864 * 2.0**-24 * magnitude
     assert err.max() <= 2e-3 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("shape, layers, times", [((4, 64, 128, 128), (0, 5), 1.0), ((8, 1024, 8, 8), (0, 1, 5), 1.6)])
+def test_weight_gradients_round_like_row_sums(fm, shape, layers, times):
+    """Rounding of the weight gradients: no worse than FP32 sums by rows, of the rows of a plane, and FP64 over the planes.
+    The network is one whose gradients have exactly known operands: the input layer reads one voxel and channel, the
+    blocks add a constant, the output layer reads one voxel, so that g = bf16(dy w) and every activation follow on the
+    host, and the error is that of the sums alone.  With rows of 32 voxels and S steps of rows a block the variance is
+    (32 + S) / (W + H) of the row sums' (0.61 of their error at 4 x 64 x 128 x 128, S = 64; one chain over a block would
+    have 2.8 times it; in the input layer, whose products have 16 bits, short row sums are exact and the two are near
+    each other).  In small planes both add a few rows and matrix instructions that truncate may double the variance (1.4
+    times; partial sums over the 8 planes that a cap of 1024 rows gives: more than 2)."""
+    rng = np.random.default_rng(5)
+    bf = lambda a: onet.bf16(np.asarray(a, np.float32)).astype(np.float32)
+    params = [[np.zeros(ws, np.float32), np.zeros(bs, np.float32)] for ws, bs in onet.param_shapes()]
+    w1, w6 = bf(rng.uniform(0.2, 1.0, 32)), bf(rng.uniform(0.2, 1.0, 32))
+    params[0][0].reshape(27, 32, 2)[13, :, 0] = w1
+    params[5][0].reshape(27, 32)[13] = w6
+    for l in range(5):
+        params[l][1][...] = bf(rng.uniform(0.05, 0.3, 32))
+    x = bf(rng.uniform(0.0, 1.0, shape + (2,)))
+    net = fm.Net(1)
+    net.set_params(flat(params))
+    dx = fm.DeviceArray.from_host(fm.to_bf16_bits(x))
+    d = fm.DeviceArray(shape, np.float32)
+    net.forward(dx, shape, d)
+    fm.device_synchronize()
+    y = d.download()
+    t = (y - rng.normal(0.0, 1.0, shape)).astype(np.float32)
+    dy = (2.0 * (y.astype(np.float64) - t) / t.size).astype(np.float32)
+    net.backward(dx, fm.DeviceArray.from_host(t), shape)
+    got = unflat(net.grads())
+
+    def activation(c, layer):  # channel c of the layer's output
+        h = bf(params[0][1][c] + x[..., 0] * w1[c])
+        for l in range(1, layer + 1):
+            h = bf(h + params[l][1][c])
+        return h
+
+    def row_sums(p):  # FP32 along the rows, then along the columns, FP64 over the planes
+        s = np.cumsum(np.cumsum(p, -1, dtype=np.float32)[..., -1], -1, dtype=np.float32)[..., -1]
+        return s.sum(dtype=np.float64)
+
+    g = [bf(dy * w) for w in w6]
+    for l in layers:
+        a = [np.ascontiguousarray(x[..., i]) for i in range(2)] if l == 0 else [activation(c, l - 1) for c in range(32)]
+        if l == 1:  # 32 x 32 pairs: a few of them
+            a = a[:8]
+        gpu, ref = [], []
+        for co, gv in enumerate(g if l < 5 else [dy]):
+            for ci, av in enumerate(a):
+                exact = np.dot(gv.reshape(-1).astype(np.float64), av.reshape(-1).astype(np.float64))
+                gpu.append(got[l][0].reshape(27, -1, len(a) if l != 1 else 32)[13, co, ci] - exact)
+                ref.append(row_sums(gv * av) - exact)
+        rms = [float(np.sqrt(np.mean(np.square(e)))) for e in (gpu, ref)]
+        print(f"{shape} layer {l + 1}: error {rms[0]:.2e}, row sums {rms[1]:.2e}", flush=True)
+        assert rms[0] <= times * rms[1], (l, rms)
