@@ -192,6 +192,7 @@ constexpr unsigned kBoxSuper = 4;  // supertiles of 4^3 cubes, about 1.7 MB of s
 
 struct BoxMap {
     double guard;
+    int span[3];        // the cubes' extents less one: kT - 1, or less of a target less than kT wide
     int ny, nz;         // rows and planes of the box
     int pieces;         // pieces staged per row
     int pitch, plane;   // bytes from row to row and plane to plane
@@ -253,7 +254,7 @@ __global__ __launch_bounds__(kBoxThreads, 4) void transform_box_kernel(const S* 
     for (int a = 0; a < 3; ++a) {
         double r = fma(M.m[4 * a], (double)x0, fma(M.m[4 * a + 1], (double)y0, fma(M.m[4 * a + 2], (double)zb, M.m[4 * a + 3])));
 #pragma unroll
-        for (int k = 0; k < 3; ++k) r += fmin(M.m[4 * a + k] * (kT - 1), 0.0);
+        for (int k = 0; k < 3; ++k) r += fmin(M.m[4 * a + k] * (double)B.span[k], 0.0);
         org[a] = __builtin_amdgcn_readfirstlane((int)floor(r - 1e-5));
     }
     constexpr int n = sizeof(P) / sizeof(S);
@@ -409,17 +410,26 @@ static double transform_guard(const Mat12& M, int tw, int th, int zend, double r
 // The box kernel where its box fits 64 KiB of LDS, so that one workgroup of a
 // CU computes while another stages, and where the guard leaves few samples to
 // evaluate twice (coordinates up to about 10^7).  Maps that shrink the
-// source by more than about 2 take the general kernel.
+// source by more than about 2 take the general kernel, and so do one or two planes, which
+// leave a workgroup little to compute behind its staging (512 x 512 voxels under
+// rotations to 45 degrees, us, general and box: one plane 6.5, 10.4; two 8.5 to 10.0, 11.0 to 11.4;
+// three 11.1 to 13.1, 11.2 to 11.9; eight 22 to 31, 14 to 19).
 template <typename S, typename P>
 static bool launch_box(const S* src, int w, int h, int d, S* dst, int tw, int th, int z0, int nz, const Mat12& M,
                        hipStream_t s)
 {
+    if (nz < 3) return false;
     BoxMap B;
     B.guard = transform_guard(M, tw, th, z0 + nz, 65536.0);
     if (!(B.guard < 1e-3)) return false;
+    // (a slab of a few planes, or a target that is narrower than a cube, needs less of the source:
+    // 4 planes of 1024 x 1024, 39.9 -> 36.8 us)
+    const int target[3] = {tw, th, nz};
+    for (int k = 0; k < 3; ++k) B.span[k] = std::min(kT, target[k]) - 1;
     int n[3];
     for (int a = 0; a < 3; ++a) {
-        const double e = (std::fabs(M.m[4 * a]) + std::fabs(M.m[4 * a + 1]) + std::fabs(M.m[4 * a + 2])) * (kT - 1);
+        double e = 0.0;
+        for (int k = 0; k < 3; ++k) e += std::fabs(M.m[4 * a + k]) * B.span[k];
         if (!(e < 140.0)) return false;
         n[a] = (int)std::ceil(e + 1e-4) + 2;
     }

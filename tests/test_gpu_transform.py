@@ -147,3 +147,25 @@ def test_transform_box_edges(fm, orc, bits, shape, tshape, angles, scale):
     fm.device_synchronize()
     want = orc.transform(src.astype(np.uint16), M, tshape, bits=bits).astype(src.dtype)
     assert np.array_equal(from_device(ddst, src.dtype), want)
+
+
+def check_bit_exact(fm, orc, src, tshape, M, bits):
+    dsrc, ddst = to_device(src), empty_device(tshape, src.dtype)
+    fm.transform_device(dsrc.ptr, src.shape, ddst.ptr, tshape, np.asarray(M, np.float32), bits=bits)
+    fm.device_synchronize()
+    want = orc.transform(src.astype(np.uint16), np.asarray(M, np.float32), tshape, bits=bits).astype(src.dtype)
+    got = from_device(ddst, src.dtype)
+    assert np.array_equal(got, want), (int(np.count_nonzero(got != want)), np.argwhere(got != want)[:4])
+    return want
+
+
+@pytest.mark.parametrize("bits", [16, 8])
+@pytest.mark.parametrize("tshape", [(1, 40, 50), (2, 17, 33), (5, 16, 16), (15, 20, 70), (17, 3, 40), (33, 1, 1), (40, 5, 2),
+                                    (1, 1, 100), (1, 70, 1)])
+def test_transform_thin_targets(fm, orc, bits, tshape):
+    """Targets of fewer than 16 voxels along an axis: the staged box covers the voxels there are."""
+    for shape in ((36, 48, 64), (35, 47, 61)):
+        src = volume(shape, bits, seed=sum(tshape) + bits)
+        for angles, scale in (((0, 0, 0), 1.0), ((20, -30, 40), 1.2), ((0, 90, 0), 1.0)):
+            want = check_bit_exact(fm, orc, src, tshape, rotated(angles, scale, shape, tshape), bits)
+            assert want.any()
