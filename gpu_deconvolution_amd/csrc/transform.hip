@@ -260,6 +260,17 @@ __global__ __launch_bounds__(kBoxThreads, 4) void transform_box_kernel(const S* 
     constexpr int n = sizeof(P) / sizeof(S);
     if constexpr (sizeof(P) == 16) org[0] &= -n;  // rows are staged from 16-byte boundaries
 
+    // wavefront: 16 x 4 columns, 8 planes
+    const int x = x0 + (int)(threadIdx.x & 15), y = y0 + (int)(threadIdx.x >> 4 & 15), zw = zb + (int)(threadIdx.x >> 8) * 8;
+    S* out = dst + ((size_t)(zw - z0) * th + y) * tw + x;
+    const size_t pstride = (size_t)th * tw;
+    // a box that meets no texel: its samples are zero (uniform)
+    if (org[0] >= w || org[0] + B.pieces * n <= 0 || org[1] >= h || org[1] + B.ny <= 0 || org[2] >= d || org[2] + B.nz <= 0) {
+        if (x < tw && y < th)
+            for (int z = zw; z < min(zw + 8, ze); ++z, out += pstride) *out = 0;
+        return;
+    }
+
     // Staging: a thread takes piece q of the rows row, row + step, ... (iy, iz by
     // counting), four loads in flight; past the last row, and in the threads left
     // over, it repeats a row.
@@ -315,8 +326,6 @@ __global__ __launch_bounds__(kBoxThreads, 4) void transform_box_kernel(const S* 
     }
     __syncthreads();
 
-    // wavefront: 16 x 4 columns, 8 planes
-    const int x = x0 + (int)(threadIdx.x & 15), y = y0 + (int)(threadIdx.x >> 4 & 15), zw = zb + (int)(threadIdx.x >> 8) * 8;
     if (x >= tw || y >= th) return;
     const double xd = (double)x, yd = (double)y, zd = (double)zw;
     double r[3];  // source coordinates, stepped from plane to plane
@@ -327,8 +336,6 @@ __global__ __launch_bounds__(kBoxThreads, 4) void transform_box_kernel(const S* 
     // byte address in LDS of texel (0, 0, 0)
     const double at0 = (double)lds_address(box) -
                        fma((double)org[2], plane, fma((double)org[1], pitch, (double)(org[0] * (int)sizeof(S))));
-    S* out = dst + ((size_t)(zw - z0) * th + y) * tw + x;
-    const size_t pstride = (size_t)th * tw;
     double worst = 0.0;  // largest distance of an unrounded sample from its rounded value
     auto sample = [&]() -> S {
         const double fx = floor(r[0]), fy = floor(r[1]), fz = floor(r[2]);

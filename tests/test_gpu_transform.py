@@ -169,3 +169,19 @@ def test_transform_thin_targets(fm, orc, bits, tshape):
         for angles, scale in (((0, 0, 0), 1.0), ((20, -30, 40), 1.2), ((0, 90, 0), 1.0)):
             want = check_bit_exact(fm, orc, src, tshape, rotated(angles, scale, shape, tshape), bits)
             assert want.any()
+
+
+@pytest.mark.parametrize("bits", [16, 8])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+def test_transform_boxes_beside_the_volume(fm, orc, bits, axis):
+    """Boxes that lie outside the volume, touch it, or hold its last texel only, on either side of an axis."""
+    tshape = (33, 35, 37)
+    for shape in ((20, 24, 32), (19, 23, 29)):
+        src = volume(shape, bits, seed=axis + bits)
+        n, t = shape[::-1][axis], tshape[::-1][axis]
+        seen = []
+        for shift in (-3e4, -t - 1.0, -t, -t + 0.5, -t + 1.0, -17.0, -16.5, -15.5, n - 17.0, n - 1.0, n - 0.25, n, n + 1.0, 3e4, 1e7):
+            M = IDENT.copy()
+            M[axis, 3] = shift
+            seen.append(check_bit_exact(fm, orc, src, tshape, M, bits).any())
+        assert any(seen) and not all(seen)
