@@ -188,7 +188,7 @@ __global__ __launch_bounds__(256) void transform_general_kernel(const S* __restr
 // so a sample farther than that from a rounding boundary is the definition's, and
 // any other is evaluated by transform_sample.
 constexpr int kT = 16, kBoxThreads = 512;
-constexpr unsigned kBoxSuper = 4;  // supertiles of 4^3 cubes, about 1.7 MB of source
+constexpr unsigned kBoxSuper = 4;  // supertiles of 4^3 cubes, about 1.7 MB of source; flat targets' of fewer layers
 
 struct BoxMap {
     double guard;
@@ -199,6 +199,7 @@ struct BoxMap {
     int step, step_y, step_z;  // rows staged at a time: floor(threads / pieces) = step_z ny + step_y
     unsigned magic_pieces;     // ceil(2^16 / pieces): i / pieces = i magic >> 16 for i < 512, pieces <= 150
     unsigned nx, nby, nsx, nsy;  // cubes, and supertiles, along x and y
+    unsigned sz;                 // cubes of a supertile along z
 };
 
 __device__ __forceinline__ double lerp(double a, double b, double f) { return fma(f, b - a, a); }
@@ -241,9 +242,9 @@ __global__ __launch_bounds__(kBoxThreads, 4) void transform_box_kernel(const S* 
 {
     extern __shared__ __attribute__((aligned(16))) char box[];
     constexpr unsigned s = kBoxSuper;
-    const unsigned lid = xcd_block(blockIdx.x, gridDim.x), st = lid / (s * s * s), wi = lid % (s * s * s);
+    const unsigned lid = xcd_block(blockIdx.x, gridDim.x), st = lid / (s * s * B.sz), wi = lid % (s * s * B.sz);
     const unsigned bx = st % B.nsx * s + wi % s, by = st / B.nsx % B.nsy * s + wi / s % s,
-                   bz = st / (B.nsx * B.nsy) * s + wi / (s * s);
+                   bz = st / (B.nsx * B.nsy) * B.sz + wi / (s * s);
     const int x0 = (int)bx * kT, y0 = (int)by * kT, zb = z0 + (int)bz * kT, ze = z0 + nz;
     if (bx >= B.nx || by >= B.nby || zb >= ze) return;
 
@@ -420,7 +421,7 @@ static double transform_guard(const Mat12& M, int tw, int th, int zend, double r
 // source by more than about 2 take the general kernel, and so do one or two planes, which
 // leave a workgroup little to compute behind its staging (512 x 512 voxels under
 // rotations to 45 degrees, us, general and box: one plane 6.5, 10.4; two 8.5 to 10.0, 11.0 to 11.4;
-// three 11.1 to 13.1, 11.2 to 11.9; eight 22 to 31, 14 to 19).
+// three 11.1 to 13.1, 11.2 to 11.9; eight 22 to 31, 14 to 19; of 1024 x 1024 three 27, 23).
 template <typename S, typename P>
 static bool launch_box(const S* src, int w, int h, int d, S* dst, int tw, int th, int z0, int nz, const Mat12& M,
                        hipStream_t s)
@@ -430,7 +431,7 @@ static bool launch_box(const S* src, int w, int h, int d, S* dst, int tw, int th
     B.guard = transform_guard(M, tw, th, z0 + nz, 65536.0);
     if (!(B.guard < 1e-3)) return false;
     // (a slab of a few planes, or a target that is narrower than a cube, needs less of the source:
-    // 4 planes of 1024 x 1024, 39.9 -> 36.8 us)
+    // 3 planes of 1024 x 1024: 36 -> 23 us together with the layers below; the general kernel 27)
     const int target[3] = {tw, th, nz};
     for (int k = 0; k < 3; ++k) B.span[k] = std::min(kT, target[k]) - 1;
     int n[3];
@@ -456,10 +457,12 @@ static bool launch_box(const S* src, int w, int h, int d, S* dst, int tw, int th
     B.nx = (unsigned)((tw + kT - 1) / kT);
     B.nby = (unsigned)((th + kT - 1) / kT);
     const unsigned nbz = (unsigned)((nz + kT - 1) / kT);
+    // (no empty layers: 8 planes of 1024 x 1024 took 42 us with three of them launched, 29 without)
+    B.sz = std::min(kBoxSuper, nbz);
     B.nsx = (B.nx + kBoxSuper - 1) / kBoxSuper;
     B.nsy = (B.nby + kBoxSuper - 1) / kBoxSuper;
     const unsigned long long blocks =
-        (unsigned long long)B.nsx * B.nsy * ((nbz + kBoxSuper - 1) / kBoxSuper) * kBoxSuper * kBoxSuper * kBoxSuper;
+        (unsigned long long)B.nsx * B.nsy * ((nbz + B.sz - 1) / B.sz) * kBoxSuper * kBoxSuper * B.sz;
     if (blocks > 0x7fffffffull || (double)w * h * sizeof(S) * B.nz >= 4294967296.0) return false;
     launch(transform_box_kernel<S, P>, dim3((unsigned)blocks), dim3(kBoxThreads), (unsigned)lds, s, src, w, h, d, dst, tw,
            th, z0, nz, M, B);
