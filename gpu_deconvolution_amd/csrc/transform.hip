@@ -462,6 +462,13 @@ static bool launch_box(const S* src, int w, int h, int d, S* dst, int tw, int th
     B.plane = (B.ny | 1) * B.pitch;
     const size_t lds = (size_t)B.plane * B.nz + 16;  // (a row's last read reaches 8 bytes past it)
     if (lds > 64 * 1024) return false;
+    // 16-bit rows off the 16-byte boundaries, in a box of which only two workgroups fit a CU (160 KiB of
+    // LDS): staging in 4-byte pieces is then slower than the general kernel where the 64 lanes of its
+    // wavefront stay on few source rows (512 x 384 x 64 voxels from 1021 x 768 x 128, us, general and
+    // box: unrotated at scale 1.7, 48.7 KB, 67, 66; at 1.8, 55.8 KB, 67, 90; turned by 3 degrees about each
+    // axis at 1.7, 65.4 KB, 69, 93; but by 45 degrees about z at 1.5, 59.5 KB, 146, 93).  8 bits: 91, 85.
+    if (sizeof(S) == 2 && sizeof(P) == 4 && 3 * lds > 160 * 1024 && std::fabs(M.m[4]) + std::fabs(M.m[8]) < 0.7)
+        return false;
     B.step = kBoxThreads / B.pieces;
     B.step_z = B.step / B.ny;
     B.step_y = B.step % B.ny;

@@ -217,3 +217,14 @@ def test_transform_ties_take_the_definition(fm, orc, bits, frac, shape, depth):
     M = IDENT.copy()
     M[:, 3] = frac
     check_bit_exact(fm, orc, src, tshape, M, bits)
+
+
+@pytest.mark.parametrize("angles, scale", [((0, 0, 0), 1.7), ((0, 0, 0), 1.75), ((0, 0, 0), 1.9), ((3, 3, 3), 1.7), ((0, 0, 45), 1.5),
+                                           ((0, 0, 20), 1.65), ((0, 0, 25), 1.65)])
+@pytest.mark.parametrize("bits", [16, 8])
+def test_transform_large_boxes_of_odd_rows(fm, orc, bits, angles, scale):
+    """Boxes on both sides of 160 / 3 KiB with rows off the 16-byte boundaries, along and across the source rows."""
+    shape, tshape = (60, 65, 77), (33, 37, 41)
+    src = volume(shape, bits, seed=int(10 * scale) + bits)
+    want = check_bit_exact(fm, orc, src, tshape, rotated(angles, scale, shape, tshape), bits)
+    assert (want > 0).mean() > 0.3
