@@ -192,14 +192,14 @@ constexpr unsigned kBoxSuper = 4;  // supertiles of 4^3 cubes, about 1.7 MB of s
 
 struct BoxMap {
     double guard;
-    int span[3];        // the cubes' extents less one: kT - 1, or less of a target less than kT wide
+    double low[3];      // least source coordinate of a cube, from its first voxel's, less a margin for rounding
     int ny, nz;         // rows and planes of the box
     int pieces;         // pieces staged per row
     int pitch, plane;   // bytes from row to row and plane to plane
     int step, step_y, step_z;  // rows staged at a time: floor(threads / pieces) = step_z ny + step_y
     unsigned magic_pieces;     // ceil(2^16 / pieces): i / pieces = i magic >> 16 for i < 512, pieces <= 150
     unsigned nx, nby, nsx, nsy;  // cubes, and supertiles, along x and y
-    unsigned sz;                 // cubes of a supertile along z
+    unsigned log_sz;             // cubes of a supertile along z
 };
 
 __device__ __forceinline__ double lerp(double a, double b, double f) { return fma(f, b - a, a); }
@@ -242,33 +242,28 @@ __global__ __launch_bounds__(kBoxThreads, 4) void transform_box_kernel(const S* 
 {
     extern __shared__ __attribute__((aligned(16))) char box[];
     constexpr unsigned s = kBoxSuper;
-    const unsigned lid = xcd_block(blockIdx.x, gridDim.x), st = lid / (s * s * B.sz), wi = lid % (s * s * B.sz);
+    const unsigned lid = xcd_block(blockIdx.x, gridDim.x), st = lid / (s * s) >> B.log_sz, wi = lid - ((st * s * s) << B.log_sz);
     const unsigned bx = st % B.nsx * s + wi % s, by = st / B.nsx % B.nsy * s + wi / s % s,
-                   bz = st / (B.nsx * B.nsy) * B.sz + wi / (s * s);
+                   bz = (st / (B.nsx * B.nsy) << B.log_sz) + wi / (s * s);
     const int x0 = (int)bx * kT, y0 = (int)by * kT, zb = z0 + (int)bz * kT, ze = z0 + nz;
     if (bx >= B.nx || by >= B.nby || zb >= ze) return;
 
-    // first texel of the box on each axis (the margin covers the coordinates'
-    // rounding; the host sized the box for it)
+    // first texel of the box on each axis
     int org[3];
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-        double r = fma(M.m[4 * a], (double)x0, fma(M.m[4 * a + 1], (double)y0, fma(M.m[4 * a + 2], (double)zb, M.m[4 * a + 3])));
-#pragma unroll
-        for (int k = 0; k < 3; ++k) r += fmin(M.m[4 * a + k] * (double)B.span[k], 0.0);
-        org[a] = __builtin_amdgcn_readfirstlane((int)floor(r - 1e-5));
+        const double r = fma(M.m[4 * a], (double)x0, fma(M.m[4 * a + 1], (double)y0, fma(M.m[4 * a + 2], (double)zb, M.m[4 * a + 3])));
+        org[a] = __builtin_amdgcn_readfirstlane((int)floor(r + B.low[a]));
     }
     constexpr int n = sizeof(P) / sizeof(S);
     if constexpr (sizeof(P) == 16) org[0] &= -n;  // rows are staged from 16-byte boundaries
 
-    // wavefront: 16 x 4 columns, 8 planes
-    const int x = x0 + (int)(threadIdx.x & 15), y = y0 + (int)(threadIdx.x >> 4 & 15), zw = zb + (int)(threadIdx.x >> 8) * 8;
-    S* out = dst + ((size_t)(zw - z0) * th + y) * tw + x;
-    const size_t pstride = (size_t)th * tw;
     // a box that meets no texel: its samples are zero (uniform)
     if (org[0] >= w || org[0] + B.pieces * n <= 0 || org[1] >= h || org[1] + B.ny <= 0 || org[2] >= d || org[2] + B.nz <= 0) {
+        const int x = x0 + (int)(threadIdx.x & 15), y = y0 + (int)(threadIdx.x >> 4 & 15);
         if (x < tw && y < th)
-            for (int z = zw; z < min(zw + 8, ze); ++z, out += pstride) *out = 0;
+            for (int z = zb + (int)(threadIdx.x >> 8); z < min(zb + kT, ze); z += kBoxThreads / 256)
+                dst[((size_t)(z - z0) * th + y) * tw + x] = 0;
         return;
     }
 
@@ -327,6 +322,8 @@ __global__ __launch_bounds__(kBoxThreads, 4) void transform_box_kernel(const S* 
     }
     __syncthreads();
 
+    // wavefront: 16 x 4 columns, 8 planes
+    const int x = x0 + (int)(threadIdx.x & 15), y = y0 + (int)(threadIdx.x >> 4 & 15), zw = zb + (int)(threadIdx.x >> 8) * 8;
     if (x >= tw || y >= th) return;
     const double xd = (double)x, yd = (double)y, zd = (double)zw;
     double r[3];  // source coordinates, stepped from plane to plane
@@ -340,6 +337,8 @@ __global__ __launch_bounds__(kBoxThreads, 4) void transform_box_kernel(const S* 
     // byte address in LDS of texel (0, 0, 0)
     const double at0 = (double)lds_address(box) -
                        fma((double)org[2], plane, fma((double)org[1], pitch, (double)(org[0] * (int)sizeof(S))));
+    S* out = dst + ((size_t)(zw - z0) * th + y) * tw + x;
+    const size_t pstride = (size_t)th * tw;
     double worst = 0.0;  // largest distance of an unrounded sample from its rounded value
     auto sample = [&]() -> S {
         const double fx = floor(r[0]), fy = floor(r[1]), fz = floor(r[2]);
@@ -363,16 +362,21 @@ __global__ __launch_bounds__(kBoxThreads, 4) void transform_box_kernel(const S* 
     }
     // Which of the 8 it was is found by computing them again: keeping the flags would cost every sample, and
     // evaluating all 8 made a wavefront wait for 8 fetches (1024^2 x 256 voxels of 8 bits shifted by
-    // (1/8, 3/8, 5/8), where 0.2 % of the samples are ties: 1570 us, 1124 here, and 1414 in the general kernel).
+    // (1/8, 3/8, 5/8), where 0.2 % of the samples are ties: 1570 us, 1010 here, and 1414 in the general kernel).
     if (!(worst < 0.5 - B.guard)) {
-        const double axy[3] = {mul_add(M.m[0], xd, M.m[1], yd), mul_add(M.m[4], xd, M.m[5], yd),
-                               mul_add(M.m[8], xd, M.m[9], yd)};
+        uint32_t tied = 0;
         first_plane();
 #pragma unroll 1
-        for (int z = zw; z < min(zw + 8, ze); ++z, out += pstride) {
+        for (int i = 0; i < min(8, ze - zw); ++i) {
             worst = 0.0;
             (void)sample();
-            if (!(worst < 0.5 - B.guard)) *out = transform_sample<S>(src, w, h, d, M, axy, z);
+            if (!(worst < 0.5 - B.guard)) tied |= 1u << i;
+        }
+        const double axy[3] = {mul_add(M.m[0], xd, M.m[1], yd), mul_add(M.m[4], xd, M.m[5], yd),
+                               mul_add(M.m[8], xd, M.m[9], yd)};
+        for (; tied; tied &= tied - 1) {
+            const int i = __builtin_ctz(tied);
+            out[i * pstride] = transform_sample<S>(src, w, h, d, M, axy, zw + i);
         }
     }
 }
@@ -445,11 +449,15 @@ static bool launch_box(const S* src, int w, int h, int d, S* dst, int tw, int th
     // (a slab of a few planes, or a target that is narrower than a cube, needs less of the source:
     // 3 planes of 1024 x 1024: 36 -> 23 us together with the layers below; the general kernel 27)
     const int target[3] = {tw, th, nz};
-    for (int k = 0; k < 3; ++k) B.span[k] = std::min(kT, target[k]) - 1;
     int n[3];
     for (int a = 0; a < 3; ++a) {
         double e = 0.0;
-        for (int k = 0; k < 3; ++k) e += std::fabs(M.m[4 * a + k]) * B.span[k];
+        B.low[a] = -1e-5;
+        for (int k = 0; k < 3; ++k) {
+            const double step = M.m[4 * a + k] * (std::min(kT, target[k]) - 1);
+            e += std::fabs(step);
+            B.low[a] += std::min(step, 0.0);
+        }
         if (!(e < 140.0)) return false;
         n[a] = (int)std::ceil(e + 1e-4) + 2;
     }
@@ -477,11 +485,13 @@ static bool launch_box(const S* src, int w, int h, int d, S* dst, int tw, int th
     B.nby = (unsigned)((th + kT - 1) / kT);
     const unsigned nbz = (unsigned)((nz + kT - 1) / kT);
     // (no empty layers: 8 planes of 1024 x 1024 took 42 us with three of them launched, 29 without)
-    B.sz = std::min(kBoxSuper, nbz);
+    B.log_sz = nbz >= 3 ? 2 : nbz - 1;
+    const unsigned sz = 1u << B.log_sz;
+    static_assert(kBoxSuper == 4);
     B.nsx = (B.nx + kBoxSuper - 1) / kBoxSuper;
     B.nsy = (B.nby + kBoxSuper - 1) / kBoxSuper;
     const unsigned long long blocks =
-        (unsigned long long)B.nsx * B.nsy * ((nbz + B.sz - 1) / B.sz) * kBoxSuper * kBoxSuper * B.sz;
+        (unsigned long long)B.nsx * B.nsy * ((nbz + sz - 1) / sz) * kBoxSuper * kBoxSuper * sz;
     if (blocks > 0x7fffffffull || (double)w * h * sizeof(S) * B.nz >= 4294967296.0) return false;
     launch(transform_box_kernel<S, P>, dim3((unsigned)blocks), dim3(kBoxThreads), (unsigned)lds, s, src, w, h, d, dst, tw,
            th, z0, nz, M, B);
