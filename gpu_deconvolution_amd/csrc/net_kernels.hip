@@ -77,17 +77,22 @@ __global__ void prep_input_kernel(const uint16_t* const* __restrict__ views, int
 // and give 32 channels: a block stages the box of kEZ x kEY x kEX voxels with its halo
 // in LDS once, and a wavefront computes rows of 32 voxels on MFMA.  Walking planes
 // would save only re-reads of the halo (0.8 dwords a voxel next to the 16 and 48 written).
+// Where the boxes are too few for the chip, several blocks (`parts`) stage one and share its rows: a
+// wavefront would else compute 16 of them in turn (24 us before boxes, 39 with one block a box, 8.7 with
+// up to 16: 2 x 16 x 32 x 32).
 constexpr int kEX = 32, kEY = 16, kEZ = 4, kEThreads = 256;
 constexpr int kEHX = kEX + 2, kEHY = kEY + 2, kEHZ = kEZ + 2, kEBox = kEHZ * kEHY * kEHX;
 
 struct EdgeTile {
-    int n, z, y, x;
+    int n, z, y, x, row;  // row: the block's first row
 };
-__device__ __forceinline__ EdgeTile edge_tile(const Geo& g)
+__device__ __forceinline__ EdgeTile edge_tile(const Geo& g, int parts)
 {
     const int nx = (g.W + kEX - 1) / kEX, ny = (g.H + kEY - 1) / kEY, nz = (g.D + kEZ - 1) / kEZ;
     int b = (int)xcd_block(blockIdx.x, gridDim.x);
     EdgeTile t;
+    t.row = b % parts * (kEThreads / 64);
+    b /= parts;
     t.x = b % nx * kEX;
     b /= nx;
     t.y = b % ny * kEY;
@@ -127,13 +132,13 @@ __device__ constexpr int box_offset(int tap) { return (tap / 9 * kEHY + tap / 3 
 // 470 here: a tap's 64 cycles of products and 64 of additions a wavefront do not overlap
 // (368 us; issuing the next tap's products first changed nothing).  At most 128 registers,
 // or the products land in accumulation registers and a copy each costs a third again (585 us).
-__global__ __launch_bounds__(kEThreads, 4) void conv_in_kernel(const uint32_t* __restrict__ x, Geo g,
+__global__ __launch_bounds__(kEThreads, 4) void conv_in_kernel(const uint32_t* __restrict__ x, Geo g, int parts,
                                                                const float* __restrict__ w,
                                                                const float* __restrict__ b,
                                                                uint16_t* __restrict__ h, uint32_t* __restrict__ relu)
 {
     __shared__ uint32_t box[2 * kEBox];  // FP32: channel 0, channel 1
-    const EdgeTile t = edge_tile(g);
+    const EdgeTile t = edge_tile(g, parts);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 31, kh = lane >> 5;
     float wk[27];
 #pragma unroll
@@ -147,7 +152,7 @@ __global__ __launch_bounds__(kEThreads, 4) void conv_in_kernel(const uint32_t* _
     });
     __syncthreads();
     const int xx = t.x + m;
-    for (int row = wave; row < kEZ * kEY; row += kEThreads / 64) {
+    for (int row = t.row + wave; row < kEZ * kEY; row += kEThreads / 64 * parts) {
         const int dz = row / kEY, dy = row % kEY, zz = t.z + dz, yy = t.y + dy;
         if (zz >= g.D || yy >= g.H) continue;  // wave-uniform
         const uint32_t* v0 = box + kh * kEBox + (dz * kEHY + dy) * kEHX + m;
@@ -396,13 +401,13 @@ __global__ void loss_kernel(const float* __restrict__ y, const float* __restrict
 // would wait for the stores of the row before it.
 // At 8 x 64 x 128 x 128 (1.68 GB moved): 719 us with a voxel per thread, whose 128 and 64 bytes
 // left in pieces, 490 here (3.4 TB/s); 554 with the masks loaded row by row.
-__global__ __launch_bounds__(kEThreads, 4) void out_dgrad_kernel(const uint32_t* __restrict__ dy, Geo g,
+__global__ __launch_bounds__(kEThreads, 4) void out_dgrad_kernel(const uint32_t* __restrict__ dy, Geo g, int parts,
                                                                  const float* __restrict__ w,
                                                                  const uint32_t* __restrict__ relu,
                                                                  float* __restrict__ dh, uint16_t* __restrict__ gout)
 {
     __shared__ uint32_t box[kEBox], mask[kEZ * kEY * kEX];
-    const EdgeTile t = edge_tile(g);
+    const EdgeTile t = edge_tile(g, parts);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), m = lane & 31, kh = lane >> 5;
     float wk[14];
     int off[14];
@@ -423,7 +428,7 @@ __global__ __launch_bounds__(kEThreads, 4) void out_dgrad_kernel(const uint32_t*
     for (int i = 0; i < kEZ * kEY * kEX / kEThreads; ++i) mask[threadIdx.x + kEThreads * i] = mk[i];
     __syncthreads();
     const int xx = t.x + m;
-    for (int row = wave; row < kEZ * kEY; row += kEThreads / 64) {
+    for (int row = t.row + wave; row < kEZ * kEY; row += kEThreads / 64 * parts) {
         const int dz = row / kEY, ry = row % kEY, zz = t.z + dz, yy = t.y + ry;
         if (zz >= g.D || yy >= g.H) continue;  // wave-uniform
         const long v = g.vox(t.n, zz, yy, xx);
@@ -554,25 +559,32 @@ void launch_pack_weights(const float* params, uint16_t* wf, uint16_t* wt, float*
     pack_weights_kernel<<<nblk(4 * kConv32, 256), 256, 0, s>>>(params, wf, wt, small);
     FMVD_LAUNCH_CHECK();
 }
-static unsigned edge_blocks(Dims d)
+// boxes x parts: up to one residency of the chip (four blocks a CU), a row a wavefront at least
+static unsigned edge_blocks(Dims d, int* parts)
 {
     const long n = (long)d.N * ((d.D + kEZ - 1) / kEZ) * ((d.H + kEY - 1) / kEY) * ((d.W + kEX - 1) / kEX);
     if (n > 0x7fffffffL) throw_msg("network: volume too large");
-    return (unsigned)n;
+    *parts = (int)std::clamp<long>(1024 / n, 1, kEZ * kEY / (kEThreads / 64));
+    return (unsigned)(n * *parts);
 }
 void launch_conv_in(const uint16_t* x, Dims d, const float* small, const float* params, uint16_t* h,
                     uint32_t* relu, hipStream_t s)
 {
-    conv_in_kernel<<<edge_blocks(d), kEThreads, 0, s>>>(reinterpret_cast<const uint32_t*>(x), geo(d), small,
-                                                        params + off_b(0), h, relu);
+    int parts;
+    const unsigned blocks = edge_blocks(d, &parts);
+    conv_in_kernel<<<blocks, kEThreads, 0, s>>>(reinterpret_cast<const uint32_t*>(x), geo(d), parts, small,
+                                                params + off_b(0), h, relu);
     FMVD_LAUNCH_CHECK();
 }
 void launch_conv_out(const uint16_t* h, const uint16_t* x, Dims d, const float* small, const float* params, float* y,
                      bool training, hipStream_t s)
 {
-    // segments of about 16 planes: a segment reads two planes beyond its ends
-    const int nseg = (d.D + 15) / 16;
-    const long blocks = (long)d.N * ((d.H + kOY - 1) / kOY) * ((d.W + kOX - 1) / kOX) * nseg;
+    // segments of about 16 planes: a segment reads two planes beyond its ends; of fewer planes
+    // where the blocks would leave CUs idle (2 x 16 x 32 x 32: 69 us in one segment, 16 so;
+    // in every voxel on its own 14)
+    const long columns = (long)d.N * ((d.H + kOY - 1) / kOY) * ((d.W + kOX - 1) / kOX);
+    const int planes = (int)std::clamp<long>((columns * d.D + 511) / 512, 1, 16), nseg = (d.D + planes - 1) / planes;
+    const long blocks = columns * nseg;
     if (blocks > 0x7fffffffL) throw_msg("network: volume too large");
     (training ? conv_out_kernel : conv_out_mfma_kernel)<<<(unsigned)blocks, kOThreads, 0, s>>>(
         h, reinterpret_cast<const uint32_t*>(x), geo(d), small + 27 * 64, params + off_b(5), y, nseg);
@@ -588,8 +600,10 @@ int launch_loss(const float* y, const float* t, long count, float* dy, double* p
 void launch_out_dgrad(const float* dy, Dims d, const float* small, const uint32_t* relu, float* dh, uint16_t* gout,
                       hipStream_t s)
 {
-    out_dgrad_kernel<<<edge_blocks(d), kEThreads, 0, s>>>(reinterpret_cast<const uint32_t*>(dy), geo(d), small + 27 * 64,
-                                                          relu, dh, gout);
+    int parts;
+    const unsigned blocks = edge_blocks(d, &parts);
+    out_dgrad_kernel<<<blocks, kEThreads, 0, s>>>(reinterpret_cast<const uint32_t*>(dy), geo(d), parts, small + 27 * 64,
+                                                  relu, dh, gout);
     FMVD_LAUNCH_CHECK();
 }
 void launch_adam(float* p, const float* g, float* m, float* v, int count, float lr, int step, hipStream_t s)

@@ -261,3 +261,28 @@ def test_weight_gradients_round_like_row_sums(fm, shape, layers, times):
         rms = [float(np.sqrt(np.mean(np.square(e)))) for e in (gpu, ref)]
         print(f"{shape} layer {l + 1}: error {rms[0]:.2e}, row sums {rms[1]:.2e}", flush=True)
         assert rms[0] <= times * rms[1], (l, rms)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (2, 16, 32), (5, 17, 33), (16, 40, 64), (18, 9, 40), (33, 47, 95)])
+def test_few_boxes_are_shared_by_blocks(fm, shape):
+    """Volumes of few boxes and columns, whose rows and planes are dealt to more blocks, give the bits that they have
+    among the voxels of a larger batch, which takes one block a box and segments of 16 planes.  The small volume is the
+    first sample of that batch."""
+    n = -(-2100 * 2048 // int(np.prod(np.ceil(np.array(shape) / (4, 16, 32)) * (4, 16, 32))))
+    params, x, _ = make_problem(3, (2,) + shape)
+    net = fm.Net(1)
+    net.set_params(flat(params))
+    for many in (1, min(n, 2100)):
+        xs = np.concatenate([x] + [x[:1]] * max(0, many - 2))[:many]
+        y = fm.DeviceArray((many,) + shape, np.float32)
+        net.forward(fm.DeviceArray.from_host(fm.to_bf16_bits(xs)), (many,) + shape, y)
+        fm.device_synchronize()
+        if many == 1:
+            one = y.download()[0]
+    assert np.array_equal(one, y.download()[0])
+    view = np.random.default_rng(2).integers(1, 9, shape).astype(np.uint16)
+    est = fm.DeviceArray(shape, np.float32)
+    net.infer([fm.DeviceArray.from_host(view)], 1.0, est, floor_value=-1e30)
+    x = onet.bf16(np.stack([view, view], -1).astype(np.float64))
+    want, _ = onet.forward(params, x, quant=True)
+    assert relL2(est.download(), want) < 2e-2
