@@ -221,11 +221,11 @@ def streamed_leg(fm, synth, seed=1001, iters=30):
     assert out.shape == shape
     rate = V * Z * H * W * iters / el
     log(f"[bench] streamed 1024^2 x 512: {iters} iterations in {el:.2f}s -> {rate:.4g} view-voxel it/s "
-        f"(batch {info['batch']}, chunk {info['chunk']})")
+        f"(batch {info['stream_batch']}, chunk {info['chunk']})")
     return {"workload": f"4 views 1024x1024x512 uint16, 20k beads, random affines, 41x41 PSFs, {iters} iterations "
                         f"through fmvd_deconvolve_planes_cuda_16 from host planes (FFT {info['fft_h']}x{info['fft_w']})",
             "value": rate, "unit": "view-voxel RL iterations/s", "seconds": el, "pcie_inclusive": True,
-            "batch_planes": info["batch"], "planes_per_launch": info["chunk"]}
+            "batch_planes": info["stream_batch"], "planes_per_launch": info["chunk"]}
 
 
 def batched_workload(fm, synth, seed=2024, nvol=48, iters=25, kernel=31):

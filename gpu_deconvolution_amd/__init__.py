@@ -95,6 +95,8 @@ def lib() -> C.CDLL:
                                                C.POINTER(vp), i, i, vp, vp, vp]),
         "fmvd_plan_info_cuda_16": (i, [vp, C.POINTER(C.c_int)]),
         "fmvd_plan_info_cuda_8": (i, [vp, C.POINTER(C.c_int)]),
+        "fmvd_stream_planes_cuda_16": (i, [vp]),
+        "fmvd_stream_planes_cuda_8": (i, [vp]),
         "fmvd_snap_transform_size": (i, [i]),
         "fmvd_fft_extent_supported": (i, [i, i]),
         "fmvd_kernel_timing_enable": (None, [i]),
@@ -246,7 +248,9 @@ class Deconvolver:
     def info(self) -> dict:
         d = (C.c_int * 7)()
         self._info(self.plan, d)
-        return dict(data_h=d[0], data_w=d[1], fft_h=d[2], fft_w=d[3], views=d[4], batch=d[5], chunk=d[6])
+        stream = lib().fmvd_stream_planes_cuda_16 if self.bits == 16 else lib().fmvd_stream_planes_cuda_8
+        return dict(data_h=d[0], data_w=d[1], fft_h=d[2], fft_w=d[3], views=d[4], batch=d[5], chunk=d[6],
+                    stream_batch=stream(self.plan))
 
     def set_batch_planes(self, n: int) -> int:
         return self._set_batch(self.plan, int(n))

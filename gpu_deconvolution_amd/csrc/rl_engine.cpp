@@ -572,10 +572,13 @@ template <typename S> struct Plan {
     }
 
     // Planes per batch of the streaming pipeline: one chunk (the launches of a
-    // larger batch are no larger), so that a short stream already overlaps its
-    // host copies with the device, unless the caller set the batch.
+    // larger batch are no larger), so that streams of several chunks overlap their
+    // host copies with the device, unless the caller set the batch or a look-ahead.
+    // (A chunk is 8 planes at FFT 1536^2 and 16 at 512^2, but 256 at 256^2: shorter streams
+    // are one batch.)
     int stream_planes() const
     {
+        if (lookahead > 0) return lookahead;
         return batchCap > 0 ? batchCap : std::min(batch_planes(), std::max(chunk_planes(), nStreams));
     }
 
@@ -905,6 +908,9 @@ int fmvd_set_batch_planes_cuda_8(struct fmvd_plan_cuda_8* plan, int planes)
     plan->impl.batchCap = planes > 0 ? planes : 0;
     return plan->impl.batch_planes();
 }
+
+int fmvd_stream_planes_cuda_16(const struct fmvd_plan_cuda_16* plan) { return plan ? plan->impl.stream_planes() : -1; }
+int fmvd_stream_planes_cuda_8(const struct fmvd_plan_cuda_8* plan) { return plan ? plan->impl.stream_planes() : -1; }
 
 int fmvd_set_chunk_planes_cuda_16(struct fmvd_plan_cuda_16* plan, int planes)
 {

@@ -102,10 +102,16 @@ int fmvd_set_estimate_sink_cuda_16(struct fmvd_plan_cuda_16 *plan, fmvd_estimate
 int fmvd_set_estimate_sink_cuda_8(struct fmvd_plan_cuda_8 *plan, fmvd_estimate_sink_t sink,
                                   void *user);
 
-/* Maximum number of planes processed together (0 = automatic, from a device
- * memory budget).  Returns the value in effect. */
+/* Maximum number of planes processed together (0 = automatic: from a device
+ * memory budget for GPU-resident volumes, one chunk for streams of host
+ * planes).  Returns the value in effect for GPU-resident volumes. */
 int fmvd_set_batch_planes_cuda_16(struct fmvd_plan_cuda_16 *plan, int planes);
 int fmvd_set_batch_planes_cuda_8(struct fmvd_plan_cuda_8 *plan, int planes);
+
+/* Planes per batch of fmvd_deconvolve_planes_cuda_* with the settings in effect
+ * (two batches are pulled before the first sink call), or the look-ahead bound. */
+int fmvd_stream_planes_cuda_16(const struct fmvd_plan_cuda_16 *plan);
+int fmvd_stream_planes_cuda_8(const struct fmvd_plan_cuda_8 *plan);
 
 /* Planes whose whole iteration chain runs before the next planes start
  * (0 = automatic: the power of two of planes whose per-iteration working
@@ -226,7 +232,8 @@ int fmvd_set_variants_cuda_16(struct fmvd_plan_cuda_16 *plan, const int *variant
 int fmvd_set_variants_cuda_8(struct fmvd_plan_cuda_8 *plan, const int *variants);
 
 /* Plan geometry: fills dims[0..6] = dataH, dataW, fftH, fftW, nViews, batch
- * planes, planes per cache-resident chunk. */
+ * planes (of a GPU-resident volume; fmvd_stream_planes_cuda_* has a stream's),
+ * planes per cache-resident chunk. */
 int fmvd_plan_info_cuda_16(const struct fmvd_plan_cuda_16 *plan, int *dims);
 int fmvd_plan_info_cuda_8(const struct fmvd_plan_cuda_8 *plan, int *dims);
 

@@ -62,3 +62,20 @@ def test_staging_kept_between_runs(fm, D):
             o, e = dec.run(planes[:n], 3, want_estimate=sink)
             assert np.array_equal(o, out[:n])
             assert not (sink and n) or np.array_equal(e, est[:n])
+
+
+@pytest.mark.parametrize("bits", [16, 8])
+def test_reported_stream_batch(fm, bits):
+    """What the plan reports as a stream's batch is what the first fill pulls: default, chunk, batch and look-ahead."""
+    D, V, dh, dw, k = 9, 1, 40, 52, 9
+    data, kernels, weights = make_case(D, V, dh, dw, k, k, bits, seed=3)
+    planes = [[data[z, v] for v in range(V)] for z in range(D)]
+    with fm.Deconvolver(dh, dw, list(weights), [x.copy() for x in kernels], bits=bits, nstreams=2, chunk_planes=4) as dec:
+        for setting, want in ((lambda: None, 4), (lambda: dec.set_chunk_planes(1), 2), (lambda: dec.set_batch_planes(3), 3),
+                              (lambda: dec.set_lookahead(5), 5)):
+            setting()
+            assert dec.info()["stream_batch"] == want
+            dec.run(planes, 1)
+            assert dec.calls.index(("put", 0)) >= want and all(c == ("get", 1) for c in dec.calls[:want])
+            if want < 5:  # the pipeline pulls a second batch behind the first, then drains
+                assert dec.calls.index(("put", 0)) == min(2 * want, D) + (2 * want > D)
