@@ -345,10 +345,11 @@ template <int N_, int T_, typename Radices, int G_ = 0, int W_ = 1, bool S_ = fa
     static constexpr int NP = Radices::count;
 };
 
-// Default plans.  Constraint: every radix divides P.  The columns per workgroup are the
-// fewest that keep a wavefront full: a smaller group waits for fewer wavefronts at its
-// barriers and ends sooner (us a launch with 256 threads, then with one wavefront: 512 x
-// 64 planes of 512 27.3, 24.8; 1024 x 32 of 1024 30.6, 28.9; 1536 x 8 of 1536 34.7, 33.8).
+// Default plans.  Constraint: every radix divides P.  At 512 to 2048 points (3072 and 3584 were not
+// measured) the columns per workgroup are the fewest that keep a wavefront full, and at 256 four: a
+// smaller group waits for fewer wavefronts at its barriers and ends sooner (us a launch with
+// 256 threads, then with one wavefront: 512 x 64 planes of 512 27.3, 24.8; 1024 x 32 of 1024 30.6, 28.9;
+// 1536 x 8 of 1536 34.7, 33.8); large launches of 1536 and 2048 points are grouped again.
 // Rows of 128 take 8 a workgroup where 16 left half of the CUs without work on one plane.
 template <int N> struct Plan;
 template <> struct Plan<8> : PlanDef<8, 1, RadixList<8>> {};

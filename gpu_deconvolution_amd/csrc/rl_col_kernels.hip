@@ -69,10 +69,24 @@ int col_variants(int H)
     return n;
 }
 
+// A plan's columns in groups of 256 threads: large launches run faster with them than with the plan's few
+// columns per workgroup, which suit launches that leave the chip room.  us a launch, few and
+// grouped: 2048 points x 28672 columns (16 planes) 111.2, 103.5; 1536 x 3072 (2 planes) 21.3, 19.6.  Times of
+// whole RL runs, few over grouped: 2048 x 1536 planes, 1 plane 0.96, 4 planes (48 MiB of spectra) 0.97 to
+// 1.03, 2048 x 4096, 2 to 8 planes 1.05; 1536 x 512, 1 plane 0.97, 1536 x 3072, 2 planes (36 MiB) 1.04,
+// 1536 x 1024 to 2560, 4 to 8 planes 0.99 to 1.02.  At 1024 points few columns win or are level.
+template <typename PL> struct Grouped : PL {
+    static constexpr int COLS = 0;
+};
+template <int H> constexpr size_t grouped_bytes() { return H == 1536 ? (size_t)32 << 20 : H == 2048 ? (size_t)64 << 20 : 0; }
+
 template <typename PL>
 static void launch_col_plan(const ColGeom& g, const float2* Xin, float2* Xout, long xstride, const float2* K,
                             int nplanes, hipStream_t s, bool conj)
 {
+    if constexpr (PL::COLS > 0 && PL::variant == 0 && grouped_bytes<PL::N>() > 0)
+        if ((size_t)nplanes * g.N * g.H * sizeof(float2) >= grouped_bytes<PL::N>())
+            return launch_col_plan<Grouped<PL>>(g, Xin, Xout, xstride, K, nplanes, s, conj);
     using C = ColCfg<PL>;
     if (g.N % C::SQ && C::T > 64) throw_msg("row count not divisible by column group");
     if (C::SQ == 1 && g.N % 2) throw_msg("single-column plans need an even column count");

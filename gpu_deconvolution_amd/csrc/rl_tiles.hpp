@@ -123,7 +123,7 @@ template <typename PL_> struct RowCfg {
     // Row lengths where that is the faster (ratio / update, us a launch, table then LDS: 512
     // 41.6 / 53.7, 38.3 / 52.2; 1024 42.6 / 53.1, 42.7 / 51.6; 1280 254.7 / 389.8,
     // 251.0 / 379.0); at 768 the further LDS reads of its four short passes cost
-    // more (46.7 / 53.9, 49.9 / 56.2), at the other lengths the two are level or so.
+    // more (46.7 / 53.9, 49.9 / 56.2), and the other lengths keep the table.
     static constexpr bool TWLDS = (N == 512 || N == 1024 || N == 1280) && tw_lds_len<PL>() > 0 && AFFINE_I && AFFINE_F;
     static constexpr int TWP = TWLDS ? tw_lds_len<PL>() : 0;
     static constexpr int TWN = TWLDS ? TWP + T : 1;
@@ -722,8 +722,10 @@ __device__ __forceinline__ void col_tile(const ColGeom& g, const float2* Xin, fl
     // The kernel column loads behind the data, ahead of the FFT, where that costs no resident
     // wavefront: us per launch over 16.8 M pixels at lengths 512, 1024, 2048 (16 values
     // per thread): 25.9 -> 24.3, 27.6 -> 25.8, 30.4 -> 29.1; with 20 (2560, 105 M pixels)
-    // 219 -> 251.  Shorter columns (256: 24.0 -> 22.5) load it where they use it: there
-    // the order changes which product of a sum is fused, and so the results' last bits.
+    // 219 -> 251.  The order of the loads can change which product of a sum the compiler fuses,
+    // and so the results' last bits: at 2048 and 4096 points it does, with the same error against 64 bits
+    // (2048 x 1024, 12 runs: 2.13e-7 either way); at 256 (24.0 -> 22.5) it would too, so
+    // shorter columns load it where they use it.
     constexpr bool EARLY_K = C::P <= 16 && C::H >= 512;
     const float2* Kr = K + (unsigned)(kx * H);
     float2 kr[EARLY_K ? C::P : 1];

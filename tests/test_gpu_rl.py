@@ -332,3 +332,20 @@ def test_autotune_cache_file(fm, tmp_path):
         assert path.read_text().splitlines() == lines
     finally:
         fm.lib().fmvd_set_autotune_cache(None)
+
+
+@pytest.mark.parametrize("dh, dw", [(2018, 994), (1506, 1506)])
+def test_grouped_columns_of_large_launches(fm, dh, dw):
+    """Column launches of 64 MiB of spectra (1536 points: 32 MiB) and more, 8 planes here, take the columns in larger groups:
+    the same bits as plane by plane."""
+    Z, V, k = 8, 1, 31
+    data, kernels, weights = make_case(Z, V, dh, dw, k, k, 16, seed=dh)
+    views, outs = [to_device(np.ascontiguousarray(data[:, v])) for v in range(V)], []
+    for chunk in (8, 1):
+        dest = empty_device((Z, dh, dw), np.float32)
+        with fm.Deconvolver(dh, dw, list(weights), [x.copy() for x in kernels], chunk_planes=chunk) as dec:
+            assert dec.info()["chunk"] == chunk and dec.info()["batch"] >= Z
+            dec.run_device([t.ptr for t in views], Z, 2, est_ptr=dest.ptr, stream=0)
+            fm.device_synchronize()
+        outs.append(from_device(dest, np.float32))
+    assert np.array_equal(*outs)
