@@ -72,8 +72,10 @@ __global__ __launch_bounds__(RowCfg<PL>::THREADS, PL::WPE) void batch_update_ker
     const int lid = (int)xcd_remap(blockIdx.x, gridDim.x);
     const int e = find_entry(list, n, lid);
     const BatchSeg& S = segs[list[e]];
-    int rg, pl;
-    grouped_tile((unsigned)(lid - list[n + e]), g.H / C::G, S.nplanes, rg, pl);
+    // (volumes of fewer planes than a group in plane order: 8 planes in two volumes 416 us a run grouped, 407 so)
+    const int local = lid - list[n + e], nrg = g.H / C::G;
+    int rg = local % nrg, pl = local / nrg;
+    if (S.nplanes >= kPlaneGroup) grouped_tile((unsigned)local, nrg, S.nplanes, rg, pl);
     const long p = S.plane0 + pl;
     update_tile<PL>(seg_geom(g, S), XE + p * xstride, XT + p * xstride, ES + p * estride, S.w[view], rg * C::G,
                     lds, twl);
