@@ -259,7 +259,7 @@ template <typename S> struct Plan {
     {
         ensure_work(np);
         const int c = std::max(1, std::min(np, chunk_planes()));
-        const int lanes = (errAcc || workX) ? 1 : (int)std::max<size_t>(1, std::min<size_t>(2, env_bytes("FMVD_LANES", 1)));
+        const int lanes = (errAcc || workX) ? 1 : lane_count();
         if (lanes > 1 && np > c) {
             if (!lane2) {
                 lane2.reset(new Stream());
@@ -277,6 +277,7 @@ template <typename S> struct Plan {
             FMVD_HIP(hipStreamWaitEvent(s, laneJoin->e, 0));
         }
     }
+    static int lane_count() { return (int)std::max<size_t>(1, std::min<size_t>(2, env_bytes("FMVD_LANES", 1))); }
     std::unique_ptr<Stream> lane2;
     std::unique_ptr<Event> laneFork, laneJoin;
     // With kernel timing on, every kTimingStride-th chunk's launches are timed.
@@ -575,11 +576,11 @@ template <typename S> struct Plan {
     // larger batch are no larger), so that streams of several chunks overlap their
     // host copies with the device, unless the caller set the batch or a look-ahead.
     // (A chunk is 8 planes at FFT 1536^2 and 16 at 512^2, but 256 at 256^2: shorter streams
-    // are one batch.)
+    // are one batch.)  Two lanes take a chunk each.
     int stream_planes() const
     {
         if (lookahead > 0) return lookahead;
-        return batchCap > 0 ? batchCap : std::min(batch_planes(), std::max(chunk_planes(), nStreams));
+        return batchCap > 0 ? batchCap : std::min(batch_planes(), std::max(lane_count() * chunk_planes(), nStreams));
     }
 
     // The pipeline's staging, two slots: kept from run to run (allocating and

@@ -79,3 +79,17 @@ def test_reported_stream_batch(fm, bits):
             assert dec.calls.index(("put", 0)) >= want and all(c == ("get", 1) for c in dec.calls[:want])
             if want < 5:  # the pipeline pulls a second batch behind the first, then drains
                 assert dec.calls.index(("put", 0)) == min(2 * want, D) + (2 * want > D)
+
+
+def test_two_lanes_in_a_stream(fm, monkeypatch):
+    """FMVD_LANES=2 runs the chunks of a stream on two streams: a batch holds one chunk for each, and results are the same."""
+    D, V, dh, dw, k = 11, 2, 40, 52, 9
+    data, kernels, weights = make_case(D, V, dh, dw, k, k, 16, seed=9)
+    planes = [[data[z, v] for v in range(V)] for z in range(D)]
+    got = []
+    for lanes, want in ((1, 2), (2, 4)):
+        monkeypatch.setenv("FMVD_LANES", str(lanes))
+        with fm.Deconvolver(dh, dw, list(weights), [x.copy() for x in kernels], nstreams=1, chunk_planes=2) as dec:
+            assert dec.info()["stream_batch"] == want
+            got.append(dec.run(planes, 3, want_estimate=True))
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
