@@ -255,7 +255,7 @@ template <typename S> struct Plan {
     }
 
     void run_batch(const S* const* views, long dstride, int np, int iterations, const float* init,
-                   long istride, S* out, float* est, long ostride, hipStream_t s, long refOffset = 0)
+                   long istride, S* out, float* est, long ostride, hipStream_t s, long refOffset = 0, int chunk0 = 0)
     {
         ensure_work(np);
         const int c = std::max(1, std::min(np, chunk_planes()));
@@ -271,7 +271,7 @@ template <typename S> struct Plan {
         }
         for (int start = 0, i = 0; start < np; start += c, ++i)
             run_chunk(views, dstride, start, std::min(c, np - start), iterations, init, istride, out, est, ostride,
-                      (lanes > 1 && (i & 1)) ? lane2->s : s, refOffset, !workX && i % kTimingStride == 0);
+                      (lanes > 1 && (i & 1)) ? lane2->s : s, refOffset, !workX && (chunk0 + i) % kTimingStride == 0);
         if (lanes > 1 && np > c) {
             FMVD_HIP(hipEventRecord(laneJoin->e, lane2->s));
             FMVD_HIP(hipStreamWaitEvent(s, laneJoin->e, 0));
@@ -280,7 +280,8 @@ template <typename S> struct Plan {
     static int lane_count() { return (int)std::max<size_t>(1, std::min<size_t>(2, env_bytes("FMVD_LANES", 1))); }
     std::unique_ptr<Stream> lane2;
     std::unique_ptr<Event> laneFork, laneJoin;
-    // With kernel timing on, every kTimingStride-th chunk's launches are timed.
+    // With kernel timing on, every kTimingStride-th chunk's launches are timed (chunk0: the
+    // chunks that the batches of the same stream before this one had).
     static constexpr int kTimingStride = 8;
 
     // The iteration chain on planes [start, start + np) of a batch.
@@ -667,7 +668,7 @@ template <typename S> struct Plan {
         };
 
         int cnt[2] = {0, 0};
-        int slot = 0;
+        int slot = 0, chunks = 0;
         cnt[0] = fill(0);
         if (cnt[0] == 0) return;
         send(0, cnt[0]);
@@ -679,7 +680,8 @@ template <typename S> struct Plan {
             for (int v = 0; v < nViews; ++v) vv[v] = staging[slot]->in.template as<S>() + (size_t)v * nb * pl;
             Staging& st = *staging[slot];
             run_batch(vv.data(), (long)pl, cnt[slot], iterations, nullptr, 0, st.out.template as<S>(),
-                      esink ? st.est.template as<float>() : nullptr, (long)pl, cs);
+                      esink ? st.est.template as<float>() : nullptr, (long)pl, cs, 0, chunks);
+            chunks += (cnt[slot] + chunk_planes() - 1) / chunk_planes();
             FMVD_HIP(hipEventRecord(st.run.e, cs));
             FMVD_HIP(hipStreamWaitEvent(down->s, st.run.e, 0));
             FMVD_HIP(hipMemcpyAsync(st.hout.p, st.out.p, sizeof(S) * pl * cnt[slot], hipMemcpyDeviceToHost, down->s));

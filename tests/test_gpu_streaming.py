@@ -93,3 +93,17 @@ def test_two_lanes_in_a_stream(fm, monkeypatch):
             assert dec.info()["stream_batch"] == want
             got.append(dec.run(planes, 3, want_estimate=True))
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
+def test_timing_stride_over_a_stream(fm):
+    """With kernel timing on, the launches of every 8th chunk of a stream are timed, also where a batch is one chunk."""
+    D, V, dh, dw, k, it = 19, 2, 40, 52, 9, 3
+    data, kernels, weights = make_case(D, V, dh, dw, k, k, 16, seed=4)
+    planes = [[data[z, v] for v in range(V)] for z in range(D)]
+    with fm.Deconvolver(dh, dw, list(weights), [x.copy() for x in kernels], nstreams=1, chunk_planes=1) as dec:
+        assert dec.info()["stream_batch"] == 1
+        with fm.KernelTiming() as kt:
+            dec.run(planes, it)
+            fm.device_synchronize()
+            assert kt.read("ratio")[1] == 3 * V * it  # chunks 0, 8, 16
+            assert kt.read("egress")[1] == 3
