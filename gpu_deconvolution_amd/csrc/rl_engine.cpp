@@ -118,10 +118,14 @@ template <typename S> struct Plan {
         return g;
     }
 
+    static size_t batch_budget() { return env_bytes("FMVD_BATCH_BYTES", (size_t)2 << 30); }
     int batch_planes() const
     {
-        if (batchCap > 0) return batchCap;
-        const size_t budget = env_bytes("FMVD_BATCH_BYTES", (size_t)2 << 30);
+        return batchCap > 0 ? batchCap : default_batch_planes();
+    }
+    int default_batch_planes() const
+    {
+        const size_t budget = batch_budget();
         const size_t per = xplane() * sizeof(float2) + eplane() * sizeof(float);
         size_t nb = budget / (per ? per : 1);
         nb = std::max<size_t>(1, std::min<size_t>(nb, 4096));
@@ -497,6 +501,8 @@ template <typename S> struct Plan {
         if (!dviews) throw_msg("d_views must not be NULL");
         const int nb = batch_planes();
         const size_t pl = plane();
+        // (staging of an earlier stream gives way to larger work buffers)
+        if (xplane() * sizeof(float2) * (size_t)std::min(nb, nplanes) > XE.bytes) release_staging();
         std::vector<const S*> vv(nViews);
         for (int start = 0; start < nplanes; start += nb) {
             const int n = std::min(nb, nplanes - start);
@@ -581,12 +587,18 @@ template <typename S> struct Plan {
     int stream_planes() const
     {
         if (lookahead > 0) return lookahead;
-        return batchCap > 0 ? batchCap : std::min(batch_planes(), std::max(lane_count() * chunk_planes(), nStreams));
+        return batchCap > 0 ? batchCap : default_stream_planes();
+    }
+    int default_stream_planes() const
+    {
+        return std::min(default_batch_planes(), std::max(lane_count() * chunk_planes(), nStreams));
     }
 
-    // The pipeline's staging, two slots: kept from run to run (allocating and
-    // pinning it on every call took 8 times as long as deconvolving 40 planes of
-    // 512^2), at most two batches of samples and results, freed with the plan.
+    // The pipeline's staging, two slots of a batch of samples and results, on the device and
+    // pinned: kept from run to run (allocating and pinning it on every call took 8 times
+    // as long as deconvolving 40 planes of 512^2) while the device's part is no larger than
+    // the batch budget or a default batch's.  Given back by set_batch, by a run on a resident volume that needs
+    // larger work buffers, and with the plan.
     struct Staging {
         DeviceBuffer in, out, est;
         PinnedBuffer hin, hout, hest;
@@ -594,6 +606,28 @@ template <typename S> struct Plan {
     };
     std::unique_ptr<Staging> staging[2];
     std::unique_ptr<Stream> down;
+    bool streaming = false;  // its buffers are in use
+
+    void release_staging()
+    {
+        if (streaming) return;
+        for (auto& st : staging) st.reset();
+    }
+    void trim_staging()
+    {
+        size_t bytes = 0;
+        for (const auto& st : staging)
+            if (st) bytes += st->in.bytes + st->out.bytes + st->est.bytes;
+        const size_t per = plane() * (sizeof(S) * (nViews + 1) + sizeof(float));
+        streaming = false;
+        if (bytes > std::max(batch_budget(), 2 * per * (size_t)default_stream_planes())) release_staging();
+    }
+    int set_batch(int planes)
+    {
+        batchCap = planes > 0 ? planes : 0;
+        release_staging();
+        return batch_planes();
+    }
 
     // fmvd_deconvolve.impl.cpp:205-300, as a double-buffered batch pipeline:
     // while batch i computes on the compute stream, the host pulls batch i+1
@@ -606,15 +640,19 @@ template <typename S> struct Plan {
         if (iterations < 0) throw_msg("negative iteration count");
         FMVD_HIP(hipSetDevice(device));
         if (lookahead > 0) return deconvolve_planes_bounded(iterations);
+        streaming = true;
         try {
             stream_batches(iterations);
         } catch (...) {
-            // no copy may be in flight on the staging that the next run fills
+            // no copy or kernel may be in flight on the staging that the next run fills
             (void)hipStreamSynchronize(copy->s);
             (void)hipStreamSynchronize(compute->s);
+            if (lane2) (void)hipStreamSynchronize(lane2->s);
             if (down) (void)hipStreamSynchronize(down->s);
+            trim_staging();
             throw;
         }
+        trim_staging();
     }
 
     void stream_batches(int iterations)
@@ -901,15 +939,13 @@ int fmvd_set_estimate_sink_cuda_8(struct fmvd_plan_cuda_8* plan, fmvd_estimate_s
 int fmvd_set_batch_planes_cuda_16(struct fmvd_plan_cuda_16* plan, int planes)
 {
     if (!plan) return -1;
-    plan->impl.batchCap = planes > 0 ? planes : 0;
-    return plan->impl.batch_planes();
+    return plan->impl.set_batch(planes);
 }
 
 int fmvd_set_batch_planes_cuda_8(struct fmvd_plan_cuda_8* plan, int planes)
 {
     if (!plan) return -1;
-    plan->impl.batchCap = planes > 0 ? planes : 0;
-    return plan->impl.batch_planes();
+    return plan->impl.set_batch(planes);
 }
 
 int fmvd_stream_planes_cuda_16(const struct fmvd_plan_cuda_16* plan) { return plan ? plan->impl.stream_planes() : -1; }

@@ -57,7 +57,9 @@ struct fmvd_plan_cuda_8;
  * (fmvd_set_chunk_planes_cuda_*) of a stream of host planes, and as many planes
  * of a GPU-resident volume as a 2 GiB device budget holds.  The staging of a stream
  * (two batches of samples and results, on the device and pinned) stays with the
- * plan. */
+ * plan while its device part is no larger than that budget or two default batches;
+ * fmvd_set_batch_planes_cuda_* gives it back, and so does a GPU-resident run
+ * that needs larger work buffers than the plan has. */
 struct fmvd_plan_cuda_16 *fmvd_initialize_cuda_16(
     int dataH, int dataW, float const *const *h_Weights, float **h_Kernel, int kernelH,
     int kernelW, fmvd_psf_type iteration_type, int nViews, int nstreams,
@@ -104,7 +106,8 @@ int fmvd_set_estimate_sink_cuda_8(struct fmvd_plan_cuda_8 *plan, fmvd_estimate_s
 
 /* Maximum number of planes processed together (0 = automatic: from a device
  * memory budget for GPU-resident volumes, one chunk for streams of host
- * planes).  Returns the value in effect for GPU-resident volumes. */
+ * planes).  Gives the staging of earlier streams back.  Returns the value in
+ * effect for GPU-resident volumes. */
 int fmvd_set_batch_planes_cuda_16(struct fmvd_plan_cuda_16 *plan, int planes);
 int fmvd_set_batch_planes_cuda_8(struct fmvd_plan_cuda_8 *plan, int planes);
 

@@ -107,3 +107,47 @@ def test_timing_stride_over_a_stream(fm):
             fm.device_synchronize()
             assert kt.read("ratio")[1] == 3 * V * it  # chunks 0, 8, 16
             assert kt.read("egress")[1] == 3
+
+
+def test_staging_is_bounded_and_given_back(fm, monkeypatch):
+    """A stream's staging stays with the plan up to the batch budget, and is given back by a new batch size and by a
+    resident run that needs larger work buffers.  Free device memory tells (batches of 64 planes of 512^2, two views:
+    two slots of 100 MB; a chunk with estimates: two of 42 MB)."""
+    V, n, k, MB = 2, 512, 9, 1 << 20
+    rng = np.random.default_rng(1)
+    planes = [[rng.integers(0, 900, (n, n)).astype(np.uint16) for _ in range(V)] for _ in range(3)]
+    kernels, weights = np.full((V, k, k), 1.0 / 81, np.float32), np.ones((V, n, n), np.float32)
+
+    def given_back(plan, batch):
+        before = fm.device_memory()[0]
+        plan.set_batch_planes(batch)
+        return fm.device_memory()[0] - before
+
+    def plan(batch=0):
+        return fm.Deconvolver(n, n, list(weights), [x.copy() for x in kernels], batch_planes=batch)
+
+    with plan(64) as dec:
+        first, _ = dec.run(planes, 2)
+        assert given_back(dec, 64) >= 190 * MB
+        again, _ = dec.run(planes, 2)
+        assert np.array_equal(first, again)
+    monkeypatch.setenv("FMVD_BATCH_BYTES", str(64 * MB))
+    with plan(64) as dec:
+        again, _ = dec.run(planes, 2)
+        assert np.array_equal(first, again)
+        assert given_back(dec, 64) < 20 * MB
+    monkeypatch.delenv("FMVD_BATCH_BYTES")
+    with plan() as dec:
+        dec.run(planes, 2, want_estimate=True)
+        assert given_back(dec, 0) >= 70 * MB
+        dec.run(planes, 2, want_estimate=True)
+        Z = 3 * dec.info()["stream_batch"]
+        views = [fm.DeviceArray((Z, n, n), np.uint16) for _ in range(V)]
+        for v in views:
+            v.fill_zero()
+        out = fm.DeviceArray((Z, n, n), np.uint16)
+        dec.run_device([v.ptr for v in views], Z, 1, out_ptr=out.ptr)
+        fm.device_synchronize()
+        assert given_back(dec, 0) < 20 * MB
+        again, _ = dec.run(planes, 2)
+        assert np.array_equal(first, again)
