@@ -77,6 +77,7 @@ struct Engine {
         if (d.N < 1 || d.D < 1 || d.H < 1 || d.W < 1) throw_msg("network: invalid volume shape");
         if (training && d.W > 256) throw_msg("network: training volume width above 256");
         const size_t nv = (size_t)d.voxels();
+        cur = Dims{0, 0, 0, 0};  // (an allocation that fails leaves no shape behind that infer could rely on)
         x.alloc(sizeof(uint16_t) * 2 * nv);
         y.alloc(sizeof(float) * nv);
         const int nh = training ? 5 : 2;

@@ -286,3 +286,17 @@ def test_few_boxes_are_shared_by_blocks(fm, shape):
     x = onet.bf16(np.stack([view, view], -1).astype(np.float64))
     want, _ = onet.forward(params, x, quant=True)
     assert relL2(est.download(), want) < 2e-2
+
+
+def test_failed_allocation_leaves_the_network_usable(fm):
+    """A volume that does not fit the device is an error; the next estimate allocates its own activations."""
+    rng = np.random.default_rng(4)
+    view = fm.DeviceArray.from_host(rng.integers(1, 900, (6, 20, 30)).astype(np.uint16))
+    a, b = fm.DeviceArray((6, 20, 30), np.float32), fm.DeviceArray((6, 20, 30), np.float32)
+    net = fm.Net(3)
+    net.infer([view], 500.0, a)
+    dummy = fm.DeviceArray((16,), np.float32)
+    with pytest.raises(fm.FmvdError):
+        net.forward(dummy, (1, 1000000, 400, 256), dummy)  # 410 GB of input alone: refused before any launch
+    net.infer([view], 500.0, b)
+    assert np.array_equal(a.download(), b.download())
