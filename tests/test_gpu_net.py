@@ -300,3 +300,17 @@ def test_failed_allocation_leaves_the_network_usable(fm):
         net.forward(dummy, (1, 1000000, 400, 256), dummy)  # 410 GB of input alone: refused before any launch
     net.infer([view], 500.0, b)
     assert np.array_equal(a.download(), b.download())
+
+
+@pytest.mark.parametrize("shape, tile", [((20, 50, 70), (8, 24, 32, 6)), ((1, 8192, 2200), None)])
+def test_tiles_with_the_reach_as_halo(fm, shape, tile):
+    """Tiles with a halo of exactly the network's reach, given and as fmvd_net_infer cuts a volume of more than 16 M voxels
+    itself: the bits of one tile."""
+    view = fm.DeviceArray.from_host(np.random.default_rng(6).integers(1, 900, shape).astype(np.uint16))
+    whole, tiled = fm.DeviceArray(shape, np.float32), fm.DeviceArray(shape, np.float32)
+    net = fm.Net(3)
+    net.infer([view], 500.0, whole, tile=shape + (6,))
+    net.infer([view], 500.0, tiled, tile=tile)
+    a, b = whole.download(), tiled.download()
+    assert np.isfinite(a).all() and a.std() > 0
+    assert np.array_equal(a, b)
