@@ -75,6 +75,7 @@ struct Engine {
     void shape(Dims d, bool training)
     {
         if (d.N < 1 || d.D < 1 || d.H < 1 || d.W < 1) throw_msg("network: invalid volume shape");
+        // (the entry points' limit: the kernels cut any width into columns of 32 voxels)
         if (training && d.W > 256) throw_msg("network: training volume width above 256");
         const size_t nv = (size_t)d.voxels();
         cur = Dims{0, 0, 0, 0};  // (an allocation that fails leaves no shape behind that infer could rely on)

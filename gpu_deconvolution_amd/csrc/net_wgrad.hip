@@ -462,21 +462,14 @@ int wgrad_blocks(Dims d)
     return (int)std::min<long>(nb, wgrad_steps(d));
 }
 
-static void check_width(Dims d)
-{
-    if (d.W > 256) throw_msg("network: volume width above 256");
-}
-
 void launch_wgrad_in(const uint16_t* g, const uint16_t* x, Dims d, float* partial, hipStream_t s)
 {
-    check_width(d);
     wgrad_in_kernel<<<wgrad_blocks(d), kWThreads, 0, s>>>(g, reinterpret_cast<const uint32_t*>(x), geo(d),
                                                           wgrad_steps(d), partial);
     FMVD_LAUNCH_CHECK();
 }
 void launch_wgrad_out(const float* dy, const uint16_t* h5, Dims d, float* partial, hipStream_t s)
 {
-    check_width(d);
     wgrad_out_kernel<<<wgrad_blocks(d), kWThreads, 0, s>>>(reinterpret_cast<const uint32_t*>(dy), h5, geo(d),
                                                            wgrad_steps(d), partial);
     FMVD_LAUNCH_CHECK();

@@ -174,13 +174,14 @@ __global__ __launch_bounds__(256) void transform_general_kernel(const S* __restr
 // cube's texels (3.8 texels an output at +-15 degrees about each axis) in LDS with
 // coalesced loads, zero outside the volume, and gathers from there without
 // bounds checks.  Gathering straight from global memory costs the texture path
-// about one cycle per lane and load, whatever the lanes' arrangement (48 L1 accesses a
+// about one cycle per lane and load, whatever the lanes' arrangement (40 L1 accesses a
 // load; 64 x 1, 32 x 2, 16 x 4 and 8 x 8 voxels ran alike, as did aligned loads):
 // 190 cycles for 64 outputs, against about 40 for the four LDS reads.  1024^2 x
-// 512 voxels of 16 bits under such maps: 3.06 ms gathered, 1.36 ms here (1.6 TB/s
-// of 2.1 GB); the VALU is about 90 % busy, 45 of the 65 instructions a sample FP64,
-// conversions or byte shifts (4.4 cycles each, the 32-bit ones 2.5).  301 x 257 x 129
-// voxels of 8 bits into 333 x 270 x 141: 95 -> 60 us.
+// 512 voxels of 16 bits under such maps: 3.06 ms gathered, 1.34 ms here (1.6 TB/s
+// of 2.1 GB).  At 2048^2 x 1024 the texture data path is busy 78 % of the time with the
+// staging, the VALU issues 63 % (74 instructions an output, most of them FP64, conversions
+// or byte shifts), the LDS is busy 38 %, a fifth of the cycles in bank conflicts.
+// 301 x 257 x 129 voxels of 8 bits into 333 x 270 x 141: 95 -> 56 us.
 //
 // The arithmetic is FP64 with fewer operations than the definition: the
 // coordinates as one FMA on a sum per (x, y) column, lerps as v + f (v' - v).  The result

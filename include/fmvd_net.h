@@ -34,7 +34,10 @@ int fmvd_net_get_params(const struct fmvd_net *net, float *host);  /* fmvd_net_p
 int fmvd_net_set_params(struct fmvd_net *net, const float *host);  /* also resets the Adam state */
 int fmvd_net_get_grads(const struct fmvd_net *net, float *host);   /* gradients of the last backward */
 
-/* d_x: bfloat16 input [N][D][H][W][2]; d_y: float [N][D][H][W] (scaled units). */
+/* d_x: bfloat16 input [N][D][H][W][2]; d_y: float [N][D][H][W] (scaled units).
+ * Forward and backward sum the output layer in one chain of FP32 FMAs a voxel, fmvd_net_infer
+ * on the matrix cores: their y may differ by FP32 rounding.  Volumes of forward and
+ * backward are at most 256 voxels wide (a limit of these entry points, not of the kernels). */
 int fmvd_net_forward(struct fmvd_net *net, const void *d_x, int N, int D, int H, int W, float *d_y, void *stream);
 /* Forward + gradients of mean((y - t)^2) over the batch (W <= 256);
  * *loss receives the loss (summed in FP64 on the GPU). */
@@ -48,8 +51,8 @@ int fmvd_net_adam(struct fmvd_net *net, float lr, void *stream);
 int fmvd_net_prep_input(const unsigned short *const *d_views, int nviews, int N, int D, int H, int W,
                         const float *d_inv_scales, void *d_x, void *stream);
 /* Warm start of one volume: d_out (float D*H*W, device) = max(scale * net(views / scale), floor_value),
- * computed tile-wise (tiles of at most 16 M voxels with the network's 6-voxel
- * reach as halo; identical to whole-volume inference).
+ * computed tile-wise (a volume of more than 16 M voxels in tiles of at most that many, with the
+ * network's 6-voxel reach as halo; identical to whole-volume inference).
  * d_views: nviews device pointers (device array). */
 int fmvd_net_infer(struct fmvd_net *net, const unsigned short *const *d_views, int nviews, int D, int H, int W,
                    float scale, float floor_value, float *d_out, void *stream);
